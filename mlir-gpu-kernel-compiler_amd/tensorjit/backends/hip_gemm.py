@@ -572,7 +572,7 @@ def tile_order_lines(ntm: int, ntn: int, group_m: int, BM: int, BN: int, vid: st
     it stays on its XCD); ``names`` / ``sfx`` name the results and temporaries."""
     T = ntm * ntn
     m, n = names
-    if group_m <= 0 or T < 2 * XCDS or T % XCDS:
+    if group_m <= 0 or T < 2 * XCDS:
         if vid is None:
             return [f"  const unsigned int {m} = blockIdx.y * {BM}u, {n} = blockIdx.x * {BN}u;"]
         return [f"  const unsigned int {m} = ({vid}) / {ntn}u * {BM}u, {n} = ({vid}) % {ntn}u * {BN}u;"]
@@ -580,9 +580,12 @@ def tile_order_lines(ntm: int, ntn: int, group_m: int, BM: int, BN: int, vid: st
     per_group = gm * ntn
     w, t, g, first, gsz, r = (f"{v}{sfx}_" for v in ("w", "t", "g", "first", "gsz", "r"))
     wid = f"blockIdx.y * {ntn}u + blockIdx.x" if vid is None else vid
+    # the first T % 8 XCDs own one tile more
+    extra = T % XCDS
+    more = f" + ({w} % {XCDS}u < {extra}u ? {w} % {XCDS}u : {extra}u)" if extra else ""
     return [
         f"  const unsigned int {w} = {wid};",
-        f"  const unsigned int {t} = ({w} % {XCDS}u) * {T // XCDS}u + {w} / {XCDS}u;",
+        f"  const unsigned int {t} = ({w} % {XCDS}u) * {T // XCDS}u{more} + {w} / {XCDS}u;",
         f"  const unsigned int {g} = {t} / {per_group}u, {first} = {g} * {gm}u;",
         f"  const unsigned int {gsz} = ({ntm}u - {first}) < {gm}u ? ({ntm}u - {first}) : {gm}u;",
         f"  const unsigned int {r} = {t} % {per_group}u;",
