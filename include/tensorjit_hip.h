@@ -44,15 +44,22 @@ extern "C" {
 
 #define TJ_HIP_ABI_VERSION 3
 
-/* Where a kernel argument points: caller input i, arena + offset, caller output j. */
-enum { TJ_ARG_INPUT = 0, TJ_ARG_ARENA = 1, TJ_ARG_OUTPUT = 2 };
+/* Where a kernel argument points: caller input i, arena + offset, caller output j, or the
+   program's workspace + offset.  The workspace holds what one launch keeps to itself (the
+   partials and tile counters of a product split over K): zero when allocated, one block per
+   stream that the program runs on (per stream and capture under stream capture, where the
+   block belongs to the captured graph's launches), one of its own for run_static, all freed
+   with the program.  The first is allocated with the program, a further stream's on its
+   first call. */
+enum { TJ_ARG_INPUT = 0, TJ_ARG_ARENA = 1, TJ_ARG_OUTPUT = 2, TJ_ARG_WORKSPACE = 3 };
 
 typedef struct tj_argref {
   int32_t kind;   /* TJ_ARG_* */
   int32_t pad_;
-  int64_t value;  /* input index, arena byte offset, or output index */
+  int64_t value;  /* input index, arena or workspace byte offset, or output index */
   int64_t bytes;  /* ARENA: size of the buffer at that offset (offset + bytes <= arena_bytes);
-                     ignored for INPUT / OUTPUT */
+                     WORKSPACE: likewise (the workspace is as large as its largest
+                     offset + bytes); ignored for INPUT / OUTPUT */
 } tj_argref;
 
 typedef struct tj_launch {

@@ -4,6 +4,7 @@
 // kernel program.  At creation each kernel argument is resolved to
 //   INPUT  i   -> i-th caller input pointer
 //   ARENA  off -> arena base + off   (intermediate placed by the memory planner)
+//   WORKSPACE off -> this stream's workspace block + off (partials of products split over K)
 //   OUTPUT j   -> j-th caller output pointer
 // and validated, so a call only fills small pointer tables and issues one
 // hipModuleLaunchKernel per kernel on the caller's stream.  The arena is a
@@ -25,6 +26,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cstdio>
@@ -105,6 +107,18 @@ struct Program {
   std::vector<KernelRec> kernels;
   char* arena = nullptr;
   size_t arena_bytes = 0;
+  // workspace blocks (TJ_ARG_WORKSPACE): one per stream and capture the program runs on, so
+  // launches of one program on several streams do not share partials or tile counters
+  struct Block {
+    hipStream_t stream;
+    unsigned long long capture;  // capture id, 0 outside stream capture
+    bool claimed;
+    char* base;
+  };
+  size_t ws_bytes = 0;
+  std::vector<Block> blocks;
+  char* static_ws = nullptr;  // the block of tj_hip_program_run_static
+  std::mutex ws_mu;
   int n_in = 0, n_out = 0;
   hipStream_t capture_stream = nullptr;
   std::list<GraphRec> graphs;  // most recently used first
@@ -124,18 +138,73 @@ struct Program {
     }
     if (capture_stream) (void)hipStreamDestroy(capture_stream);
     if (arena) (void)hipFree(arena);
+    for (Block& b : blocks) (void)hipFree(b.base);
+    if (static_ws) (void)hipFree(static_ws);
     if (module) (void)hipModuleUnload(module);
   }
 
+  // A zeroed workspace block.  Zeroed on a stream of its own, so that it also works while
+  // another stream is being captured (the caller relaxes the thread's capture mode).
+  int new_block(char** out) {
+    void* p = nullptr;
+    TJ_HIP(hipMalloc(&p, ws_bytes));
+    hipStream_t s = nullptr;
+    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipMemsetAsync(p, 0, ws_bytes, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (s) (void)hipStreamDestroy(s);
+    if (e != hipSuccess) {
+      (void)hipFree(p);
+      return hip_fail(e, "workspace block");
+    }
+    *out = static_cast<char*>(p);
+    return 0;
+  }
+
+  // The workspace block of `stream` (null when the program has no workspace).
+  int workspace_for(hipStream_t stream, char** out) {
+    *out = nullptr;
+    if (!ws_bytes) return 0;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    // the legacy stream cannot be captured, and asking it fails while another one is
+    if (stream) TJ_HIP(hipStreamGetCaptureInfo(stream, &status, &id));
+    const unsigned long long capture = status == hipStreamCaptureStatusActive ? id : 0;
+    std::lock_guard<std::mutex> lock(ws_mu);
+    for (Block& b : blocks) {
+      if (b.claimed && b.stream == stream && b.capture == capture) {
+        *out = b.base;
+        return 0;
+      }
+    }
+    for (Block& b : blocks) {
+      if (!b.claimed) {
+        b = Block{stream, capture, true, b.base};
+        *out = b.base;
+        return 0;
+      }
+    }
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    char* base = nullptr;
+    const int rc = new_block(&base);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (rc) return rc;
+    blocks.push_back(Block{stream, capture, true, base});
+    *out = base;
+    return 0;
+  }
+
   // Fill every kernel's pointer table; `base` is the arena the ARENA offsets refer to
-  // (the program's own, or the static one of tj_hip_program_run_static).
-  void bind(const void* const* in, void* const* out, char* base) {
+  // (the program's own, or the static one of tj_hip_program_run_static), `ws` the workspace.
+  void bind(const void* const* in, void* const* out, char* base, char* ws) {
     for (KernelRec& k : kernels) {
       for (size_t i = 0; i < k.refs.size(); ++i) {
         const tj_argref& r = k.refs[i];
         switch (r.kind) {
           case TJ_ARG_INPUT: k.values[i] = const_cast<void*>(in[r.value]); break;
           case TJ_ARG_ARENA: k.values[i] = base + r.value; break;
+          case TJ_ARG_WORKSPACE: k.values[i] = ws + r.value; break;
           default: k.values[i] = out[r.value]; break;
         }
       }
@@ -201,9 +270,12 @@ struct Program {
 
   // The exec for this pointer set, captured now if needed; *rec_out stays null when the
   // miss policy says to launch directly instead (only when `may_skip`).
-  int capture(const void* const* in, void* const* out, GraphRec** rec_out, bool may_skip = false) {
+  // With a workspace the exec belongs to the stream it is launched on (its launches use that
+  // stream's block).
+  int capture(const void* const* in, void* const* out, hipStream_t stream, GraphRec** rec_out, bool may_skip = false) {
     *rec_out = nullptr;
     std::vector<const void*> key = key_of(in, out);
+    if (ws_bytes) key.push_back(stream);
     if (GraphRec* hit = find(key)) {
       miss_streak = 0;
       *rec_out = hit;
@@ -214,7 +286,9 @@ struct Program {
       miss_streak++;
     }
     if (!capture_stream) TJ_HIP(hipStreamCreateWithFlags(&capture_stream, hipStreamNonBlocking));
-    bind(in, out, arena);
+    char* ws = nullptr;
+    if (int rc = workspace_for(stream, &ws)) return rc;
+    bind(in, out, arena, ws);
     GraphRec rec;
     rec.key = std::move(key);
     TJ_HIP(hipStreamBeginCapture(capture_stream, hipStreamCaptureModeThreadLocal));
@@ -390,6 +464,10 @@ int tj_hip_program_create(int device, const void* code, size_t code_size, int nk
             static_cast<uint64_t>(a.bytes) > arena_bytes - static_cast<uint64_t>(a.value))
           return fail("arena buffer [" + std::to_string(a.value) + ", +" + std::to_string(a.bytes) +
                       ") outside the " + std::to_string(arena_bytes) + "-byte arena in " + rec.name);
+      } else if (a.kind == TJ_ARG_WORKSPACE) {
+        if (a.value < 0 || a.bytes <= 0 || a.bytes > (int64_t{1} << 40) || a.value > (int64_t{1} << 40))
+          return fail("bad workspace buffer in " + rec.name);
+        p->ws_bytes = std::max(p->ws_bytes, static_cast<size_t>(a.value + a.bytes));
       } else {
         return fail("bad argument kind in " + rec.name);
       }
@@ -413,6 +491,12 @@ int tj_hip_program_create(int device, const void* code, size_t code_size, int nk
     TJ_HIP(hipMalloc(&a, arena_bytes));
     p->arena = static_cast<char*>(a);
   }
+  if (p->ws_bytes) {
+    char* b = nullptr;
+    if (int rc = p->new_block(&b)) return rc;
+    p->blocks.push_back(Program::Block{nullptr, 0, false, b});
+    if (int rc = p->new_block(&p->static_ws)) return rc;
+  }
   // tj_hip_program_run_static's arena: looked up here, where loading and allocating are
   // expected, so that entry point never makes the runtime load or place anything.  A
   // failed lookup leaves the program usable through the other entry points.
@@ -434,8 +518,11 @@ int tj_hip_program_run(void* handle, const void* const* inputs, void* const* out
   if ((p->n_in && !inputs) || (p->n_out && !outputs)) return fail("tj_hip_program_run: null pointer table");
   const uint64_t t0 = now_ns();
   DeviceScope scope(p->device);
-  p->bind(inputs, outputs, p->arena);
-  int rc = p->launch_all(static_cast<hipStream_t>(stream));
+  char* ws = nullptr;
+  int rc = p->workspace_for(static_cast<hipStream_t>(stream), &ws);
+  if (rc) return rc;
+  p->bind(inputs, outputs, p->arena, ws);
+  rc = p->launch_all(static_cast<hipStream_t>(stream));
   if (rc) return rc;
   p->stats.calls++;
   p->stats.host_ns += now_ns() - t0;
@@ -455,7 +542,7 @@ int tj_hip_program_run_static(void* handle, const void* const* inputs, void* con
                 p->static_error);
   const uint64_t t0 = now_ns();
   DeviceScope scope(p->device);
-  p->bind(inputs, outputs, p->static_base);
+  p->bind(inputs, outputs, p->static_base, p->static_ws);
   int rc = p->launch_all(static_cast<hipStream_t>(stream));
   if (rc) return rc;
   p->stats.calls++;
@@ -469,7 +556,7 @@ int tj_hip_program_capture(void* handle, const void* const* inputs, void* const*
   if ((p->n_in && !inputs) || (p->n_out && !outputs)) return fail("tj_hip_program_capture: null pointer table");
   DeviceScope scope(p->device);
   GraphRec* rec = nullptr;
-  return p->capture(inputs, outputs, &rec);
+  return p->capture(inputs, outputs, nullptr, &rec);
 }
 
 int tj_hip_program_replay(void* handle, const void* const* inputs, void* const* outputs, void* stream) {
@@ -479,13 +566,16 @@ int tj_hip_program_replay(void* handle, const void* const* inputs, void* const* 
   const uint64_t t0 = now_ns();
   DeviceScope scope(p->device);
   GraphRec* rec = nullptr;
-  int rc = p->capture(inputs, outputs, &rec, /*may_skip=*/true);
+  int rc = p->capture(inputs, outputs, static_cast<hipStream_t>(stream), &rec, /*may_skip=*/true);
   if (rc) return rc;
   if (rec) {
     TJ_HIP(hipGraphLaunch(rec->exec, static_cast<hipStream_t>(stream)));
     p->stats.graph_replays++;
   } else {
-    p->bind(inputs, outputs, p->arena);
+    char* ws = nullptr;
+    rc = p->workspace_for(static_cast<hipStream_t>(stream), &ws);
+    if (rc) return rc;
+    p->bind(inputs, outputs, p->arena, ws);
     rc = p->launch_all(static_cast<hipStream_t>(stream));
     if (rc) return rc;
     p->stats.direct_fallbacks++;
@@ -519,7 +609,9 @@ int tj_hip_kernel_time(void* handle, int k, const void* const* inputs, void* con
   if ((p->n_in && !inputs) || (p->n_out && !outputs)) return fail("tj_hip_kernel_time: null pointer table");
   DeviceScope scope(p->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  p->bind(inputs, outputs, p->arena);
+  char* ws = nullptr;
+  if (int wrc = p->workspace_for(s, &ws)) return wrc;
+  p->bind(inputs, outputs, p->arena, ws);
   KernelRec& kr = p->kernels[k];
   for (int i = 0; i < warmup; ++i)
     if (int rc = p->launch_one(kr, s)) return rc;
@@ -554,12 +646,14 @@ int tj_hip_program_time_kernels(void* handle, const void* const* inputs, void* c
   if (n == 0) return 0;
   DeviceScope scope(p->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  char* ws = nullptr;
+  if (int wrc = p->workspace_for(s, &ws)) return wrc;
   std::vector<hipEvent_t> ev(n + 1, nullptr);
   hipError_t e = hipSuccess;
   for (size_t i = 0; i <= n && e == hipSuccess; ++i) e = hipEventCreate(&ev[i]);
   int rc = 0;
   if (e == hipSuccess) {
-    p->bind(inputs, outputs, p->arena);
+    p->bind(inputs, outputs, p->arena, ws);
     e = hipEventRecord(ev[0], s);
     for (size_t k = 0; k < n && e == hipSuccess && rc == 0; ++k) {
       rc = p->launch_one(p->kernels[k], s);

@@ -37,6 +37,7 @@ from ..runtime.autotune import MatmulConfig
 from .common import access_strides, contiguous_strides, emit_expr
 from .hip_kernels import KernelGen, Launch
 from .hip_prelude import CTYPE
+from .hip_ring import ring_epilogue_lines, ring_fits, ring_loop_lines, ring_ok, ring_split_lines
 
 # (dtype, MI) -> (builtin, KI = K per instruction, KPL = K elements per lane, acc regs, operand vector type)
 MFMA = {
@@ -104,6 +105,14 @@ def config_ok(cfg: MatmulConfig, dt: DType, mm: Node | None = None) -> bool:
     _, ki, _, _, _ = MFMA[(dt, cfg.MI)]
     if cfg.PERSIST and (not cfg.DIRECT or cfg.KSPLIT > 1):
         return False
+    if cfg.STAGES:
+        ok = ring_ok(cfg, dt)
+        if ok and mm is not None:
+            M, N, K, tb = matmul_dims(mm)
+            a, b = mm.inputs
+            ok = (a.dtype == b.dtype == dt
+                  and ring_fits(cfg, dt, M, N, K, tb, math.prod(mm.shape[:-2])))
+        return ok
     if cfg.KSPLIT > 1:
         # K split over workgroups: the plain double-buffered schedule or the skinny
         # kernel, every split an equal whole number of K steps (no K edge inside a split)
@@ -655,11 +664,11 @@ def _gen_matmul(g: KernelGen, cfg: MatmulConfig, suffix: str = "") -> tuple[str,
             epi_st = None
 
     S = cfg.KSPLIT
-    ws_param = ", float* __restrict__ ws_p" if S > 1 else ""
+    ws_param = (", unsigned int* cnt_p, float* ws_p" if cfg.STAGES else ", float* __restrict__ ws_p") if S > 1 else ""
     L = [f'extern "C" __global__ __launch_bounds__({THREADS}) void {fname}({g.params()}{ws_param}) {{']
     a_bytes = 2 * BM * LDK * esz
     lds_bytes = a_bytes + 2 * BN * LDK * esz
-    if not cfg.DIRECT:
+    if not (cfg.DIRECT or cfg.STAGES):
         L.append(f"  __shared__ __attribute__((aligned(16))) char tj_lds[{lds_bytes}];")
         L.append(f"  {lds_t} (*As)[{BM}][{LDK}] = ({lds_t} (*)[{BM}][{LDK}])tj_lds;")
         L.append(f"  {lds_t} (*Bs)[{BN}][{LDK}] = ({lds_t} (*)[{BN}][{LDK}])(tj_lds + {a_bytes});")
@@ -716,6 +725,20 @@ def _gen_matmul(g: KernelGen, cfg: MatmulConfig, suffix: str = "") -> tuple[str,
         L += direct_loop_lines(cfg, M, N, K, BM, BN, TMW, TNW, KT, dvec, builtin, esz=esz)
         return _finish_matmul(L, g, k, mm, epilogue, out_shape, bidx, batch_shape, M, N, K, BM, BN, WM, WN, MI, TMW,
                               TNW, NACC, THREADS, 0, guard_m, guard_n, idx_t, cfg, dt, tb, batch, fname)
+
+    if cfg.STAGES:
+        L += ring_loop_lines(cfg, dt, M, N, K, tb, dvec, builtin)
+        meta = {"family": "matmul", "config": cfg.as_dict(), "dtype": dt.value, "M": M, "N": N, "K": K,
+                "batch": batch, "trans_b": tb, "lds_bytes": cfg.STAGES * (BM + BN) * 128 + (4 if S > 1 else 0),
+                "flops": 2.0 * M * N * K * batch, "epilogue": "lds-staged"}
+        if S > 1:
+            L += ring_split_lines(cfg, ntm, ntn, batch, "bi" if batch_shape else "0u")
+            meta.update({"split_ws": (batch * ntm * ntn * 4, batch * S * ntm * ntn * BM * BN * 4), "fused_sum": True})
+        L += ring_epilogue_lines(cfg, [o.dtype for o in k.outputs], N, M, guard_m, guard_n, idx_t,
+                                 lambda ve, cs: _run_lines(g, k, mm, epilogue, epi_inputs, out_shape, bidx, batch_shape,
+                                                           M, N, ve, cs))
+        L.append("}")
+        return "\n".join(L), Launch(fname, (ntn, ntm, batch * S), (THREADS, 1, 1), 0, meta)
 
     # K split over workgroups: this workgroup's K steps are [ksp * KTs, (ksp + 1) * KTs)
     KTs = KT // S

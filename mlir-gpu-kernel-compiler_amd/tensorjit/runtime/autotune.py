@@ -62,19 +62,20 @@ class MatmulConfig:
     DIRECT: int = 0         # 1: one wave per SIMD, tiles loaded straight into LDS (buffer_load_dwordx4 ... lds)
     KSPLIT: int = 1         # > 1: K split over that many workgroups, partials summed by the last of them
     PERSIST: int = 0        # > 0 (DIRECT only): that many workgroups (one per CU) loop over the output tiles
+    STAGES: int = 0         # > 0: ring of that many LDS stages filled by DMA (small tiles, NT and NN, any KSPLIT)
 
     def as_dict(self) -> dict:
         return {"TM": self.TM, "TN": self.TN, "TK": self.TK, "num_warps": self.num_warps,
                 "WM": self.WM, "WN": self.WN, "MI": self.MI, "SPLIT_K": self.SPLIT_K, "GROUP_M": self.GROUP_M,
                 "PINGPONG": self.PINGPONG, "INTERLEAVE": self.INTERLEAVE, "DIRECT": self.DIRECT, "KSPLIT": self.KSPLIT,
-                "PERSIST": self.PERSIST}
+                "PERSIST": self.PERSIST, "STAGES": self.STAGES}
 
     @staticmethod
     def from_dict(d: dict) -> "MatmulConfig":
         return MatmulConfig(d["TM"], d["TN"], d.get("TK", 0), d.get("num_warps", 4), d.get("WM", 2),
                             d.get("WN", 2), d.get("MI", 32), d.get("SPLIT_K", 1), d.get("GROUP_M", 8),
                             d.get("PINGPONG", 0), d.get("INTERLEAVE", 0), d.get("DIRECT", 0), d.get("KSPLIT", 1),
-                            d.get("PERSIST", 0))
+                            d.get("PERSIST", 0), d.get("STAGES", 0))
 
 
 # bf16 / fp16 candidates (MFMA 32x32x16 or 16x16x32)
@@ -84,6 +85,13 @@ HIP_CANDIDATES: list[MatmulConfig] = [
     MatmulConfig(256, 128, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1, 1, CU_COUNT),
     MatmulConfig(256, 256, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1),
     MatmulConfig(256, 128, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1),
+    # 192-row and 192-column tiles: where 256 leaves a nearly empty last round of workgroups
+    # (bf16 2000 x 11008 x 4096: 344 tiles of 256x256 187 us, 464 of 256x192 157 us)
+    MatmulConfig(256, 192, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1),
+    MatmulConfig(192, 256, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1),
+    MatmulConfig(192, 192, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1),
+    MatmulConfig(192, 128, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1),
+    MatmulConfig(128, 192, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1),
     MatmulConfig(256, 256, 64, 4, 2, 2, 32, 1, 8, 0, 0, 1),
     MatmulConfig(256, 128, 64, 4, 2, 2, 32, 1, 8, 0, 0, 1),
     # mid-size products (a few hundred 256x256 tiles or fewer): smaller direct tiles fill the CUs
@@ -152,20 +160,117 @@ HIP_F32_CANDIDATES: list[MatmulConfig] = [
 ]
 
 
+def ring_candidates(M: int, N: int, K: int, batch: int, itemsize: int) -> list[MatmulConfig]:
+    """Ring-schedule tilings of one product: the tiles below with K split over 1-12
+    workgroups, as far as the split still has work (two K tiles per part) and the grid is not
+    full without it (four workgroups per CU)."""
+    tk = 128 // itemsize
+    kt = -(-K // tk)
+    out = []
+    for tm, tn, waves, wm, wn, stages in RING_TILES:
+        if tm > 32 and tm >= 2 * M:
+            continue
+        tiles = -(-M // tm) * -(-N // tn) * batch
+        for s in (1, 2, 3, 4, 6, 8, 12):
+            if s > 1 and (tiles * s > 4 * CU_COUNT or kt < 2 * s):
+                break
+            out.append(MatmulConfig(tm, tn, tk, waves, wm, wn, 16, 1, 8, 0, 0, 0, s, 0, stages))
+    return out
+
+
+# (TM, TN, waves, WM, WN, STAGES): what 64 KiB - 144 KiB of LDS hold.  Of these the small tiles
+# win while the grid leaves CUs idle, 128x128 with 8 waves (two per SIMD, one workgroup per CU)
+# once it is full.
+RING_TILES = [
+    (32, 32, 4, 2, 2, 4), (32, 64, 4, 2, 2, 4), (32, 64, 4, 2, 2, 3), (32, 128, 4, 1, 4, 4),
+    (64, 64, 4, 2, 2, 4), (64, 64, 4, 2, 2, 3), (64, 128, 4, 2, 2, 3), (128, 64, 4, 2, 2, 3),
+    (128, 128, 8, 4, 2, 4),
+]
+
+
+def _hbm_us(M: int, N: int, K: int, batch: int, elem: int) -> float:
+    return (M * K + N * K + M * N) * batch * elem * 1e-6
+
+
+def _ring_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
+    """Microseconds of a ring-schedule product, fitted to 4.5k measured (shape, tiling) pairs
+    over 205 random decode, prompt and MLP shapes in bf16, fp16 and fp32, NT and NN (rms error
+    10% over the near-best tilings).  The busiest CU runs ``w`` workgroups, ``occ`` at a time;
+    each K tile costs its MFMAs, its DMA bytes and a latency share; HBM once; each round an
+    epilogue; a K split its partials."""
+    tm, tn, S = cfg.TM, cfg.TN, cfg.KSPLIT
+    per = -(-(-(-K // cfg.TK)) // S)
+    wgs = -(-M // tm) * -(-N // tn) * batch * S
+    occ = max(1, min(LDS_BYTES_PER_CU // (cfg.STAGES * (tm + tn) * 128 + 64), 32 // cfg.num_warps))
+    w = -(-wgs // CU_COUNT)
+    rounds, conc = -(-w // occ), min(w, occ)
+    mflop = tm * tn * cfg.TK * 2e-6 * (0.2465 if elem == 2 else 2.04) * (0.88 if cfg.num_warps == 8 else 1.0)
+    t_mfma = w * per * mflop
+    t_dma = w * per * (tm + tn) * 0.128 * 0.0085
+    t_lat = rounds * per * 0.1 / (cfg.STAGES - 1) ** 0.89
+    # weights of up to ~64 MB come from the MALL on a repeated call; more stream from HBM
+    mem = _hbm_us(M, N, K, batch, elem)
+    t_hbm = mem / 9.42
+    edge = 4.0 if N % (16 // elem) else 1.0                       # element-wise stores of ragged rows
+    t_epi = rounds * (0.62 + tm * tn * 1e-3 * 0.104 * conc * edge)
+    t_split = 1.35 + 0.02 * S * tm * tn * 0.004 * max(1.0, w / S) if S > 1 else 0.0
+    t_loop = (t_mfma ** 3.1 + t_dma ** 3.1 + t_lat ** 3.1 + t_hbm ** 3.1) ** (1 / 3.1)
+    return 1.5 + max(t_loop + rounds * per * 0.034, mem / 7.0) + t_epi + t_split
+
+
+# 16-bit direct-to-LDS tiles: (microseconds per K tile of a round with one workgroup per CU,
+# with all that fit, microseconds of a full round's epilogue), workgroups per CU; fitted to the
+# same shapes, 92 for each tile (rms error 6-13%)
+DIRECT_US = {
+    (64, 128): (0.467, 0.704, 8.9, 3), (128, 64): (0.418, 0.790, 1.5, 3), (128, 128): (0.570, 0.815, 3.0, 2),
+    (128, 192): (0.663, 1.034, 7.8, 2), (192, 128): (0.651, 1.044, 7.25, 2), (192, 192): (0.736, 0.736, 8.2, 1),
+    (192, 256): (0.818, 0.818, 12.0, 1), (256, 192): (0.817, 0.817, 11.9, 1), (256, 128): (0.751, 0.751, 6.25, 1),
+    (256, 256): (0.989, 0.989, 16.9, 1),
+}
+PERSIST_US = {(256, 256): (0.879, 25.3), (256, 128): (0.737, 9.3)}
+
+
+def _direct_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
+    """Microseconds of a direct-to-LDS product: whole rounds of ``occ`` workgroups per CU, then
+    the last round at the concurrency it has left."""
+    tm, tn = cfg.TM, cfg.TN
+    per = -(-K // cfg.TK)
+    wgs = -(-M // tm) * -(-N // tn) * batch
+    if elem == 2 and (tm, tn) in DIRECT_US:
+        one, full, epi, occ = DIRECT_US[(tm, tn)]
+        if cfg.PERSIST and (tm, tn) in PERSIST_US:
+            one = full = PERSIST_US[(tm, tn)][0]
+            epi = PERSIST_US[(tm, tn)][1]
+    else:
+        occ = 1 if cfg.PERSIST else max(1, min(LDS_BYTES_PER_CU // (2 * (tm + tn) * 128), 2))
+        mflop = tm * tn * cfg.TK * 2e-6 * (0.14 if elem == 2 else 2.0)
+        one, epi = mflop + (tm + tn) * 1e-3 * 0.396, tm * tn * 1e-3 * 0.2156 * occ
+        full = one * occ
+    if cfg.MI == 32:
+        one, full = one * 1.1, full * 1.1                         # lower clock on random data
+    if N % (16 // elem):
+        epi *= 4.0                                                # element-wise stores of ragged rows
+    rounds = -(-wgs // (CU_COUNT * occ))
+    last = -(-(wgs - (rounds - 1) * CU_COUNT * occ) // CU_COUNT)
+    step = one + (full - one) * (last - 1) / (occ - 1) if occ > 1 else full
+    t = (rounds - 1) * (per * full + epi) + per * step + epi * last / occ
+    return 1.5 + max(t, _hbm_us(M, N, K, batch, elem) / 7.0)
+
+
 def _skinny_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
-    """Streaming kernel: the B panel once from HBM, A re-read (from L2) by every
-    workgroup.  Measured on MI355X for 16 x 8192 x 8192 (TN 32, one workgroup per CU):
-    4 waves per workgroup stream B at 5.5 TB/s whatever the unroll depth (2-16 MFMA
-    steps ahead), 2 waves at 5.3, 8 waves at 4.9, 16 at 3.9; fewer workgroups than
-    CUs leave CUs idle (TN 64: 3.6 TB/s)."""
+    """Streaming kernel (M <= 16 / 32), from 35 shapes of 1-16 rows on MI355X: HBM, or rounds
+    of one workgroup per CU whose waves each run K / SPLIT_K serially (8 waves of 16 columns
+    0.83 ns per k, 4 or 2 waves of 32 columns 1.9)."""
     if M > cfg.TM or elem != 2:
         return math.inf
-    t_hbm = (M * K + N * K + M * N) * batch * elem / HBM_BYTES_PER_S
-    wgs = -(-N // cfg.TN) * batch
-    fill = min(1.0, wgs / CU_COUNT)
-    per_wave = {4: 1.0, 2: 1.04, 8: 1.13, 16: 1.4}.get(cfg.SPLIT_K, 1.5)
-    a_reads = 1.0 + cfg.TM / cfg.TN * 0.5                # A panel re-read per TN columns (from L2)
-    return t_hbm / max(fill, 1e-3) * per_wave * a_reads * 1e6
+    rounds = -(-(-(-N // cfg.TN) * batch) // CU_COUNT)
+    per_k = 0.00083 if cfg.TN == 16 else 0.0019
+    if cfg.SPLIT_K == 8 and (K // cfg.SPLIT_K) % 256:
+        per_k *= 1.3                                              # A is read in fragments, not through LDS
+    if cfg.TM == 32:
+        per_k *= 2.2
+    extra = {4: 1.0, 2: 1.04, 8: 1.06, 16: 1.1}.get(cfg.SPLIT_K, 1.2) * (1.0 if cfg.TN <= 32 else 1.05)
+    return 1.5 + max(rounds * K * per_k, _hbm_us(M, N, K, batch, elem) / 6.85) * extra
 
 
 def _sched_factor(cfg: MatmulConfig) -> float:
@@ -186,6 +291,10 @@ def _sched_factor(cfg: MatmulConfig) -> float:
 def _hip_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
     if cfg.SPLIT_K > 1:
         return _skinny_cost(cfg, M, N, K, batch, elem)
+    if cfg.STAGES:
+        return _ring_cost(cfg, M, N, K, batch, elem)
+    if cfg.DIRECT:
+        return _direct_cost(cfg, M, N, K, batch, elem)
     tm, tn, tk = cfg.TM, cfg.TN, cfg.TK or 32
     waves = cfg.num_warps
     if cfg.SPLIT_K == 1 and (tm % (cfg.WM * cfg.MI) or tn % (cfg.WN * cfg.MI)):

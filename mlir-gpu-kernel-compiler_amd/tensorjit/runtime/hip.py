@@ -16,7 +16,7 @@ LIB_NAME = "libtjhip.so"
 LIB_PATH = Path(__file__).resolve().parents[1] / LIB_NAME
 ABI_VERSION = 3
 
-INPUT, ARENA, OUTPUT = 0, 1, 2
+INPUT, ARENA, OUTPUT, WORKSPACE = 0, 1, 2, 3
 STATIC_ARENA_BYTES = 64 << 20   # TJ_HIP_STATIC_ARENA_BYTES
 
 
@@ -157,7 +157,7 @@ class NativeHipProgram:
             flat.extend(refs)
         crefs = (ArgRef * max(len(flat), 1))()
         for i, ref in enumerate(flat):
-            # (INPUT, i) / (OUTPUT, j) / (ARENA, offset, bytes)
+            # (INPUT, i) / (OUTPUT, j) / (ARENA or WORKSPACE, offset, bytes)
             crefs[i].kind, crefs[i].value = ref[0], ref[1]
             crefs[i].bytes = ref[2] if len(ref) > 2 else 0
         self._code = ctypes.create_string_buffer(code, len(code))

@@ -1,0 +1,166 @@
+"""The ring-schedule GEMM: which products it takes, and its results at the edges of tiles, of
+K tiles and of K splits, on one stream and on several."""
+import pytest
+import torch
+
+import tensorjit as tj
+from tensorjit import compiler as C
+from tensorjit.backends import hip_backend as hb
+from tensorjit.ir import DType, TensorType
+from tensorjit.runtime.autotune import RING_TILES, MatmulConfig, ring_candidates
+
+TORCH = {DType.bf16: torch.bfloat16, DType.f16: torch.float16, DType.f32: torch.float32}
+
+
+def _ring(tm, tn, waves, wm, wn, stages, split, dt):
+    return MatmulConfig(tm, tn, 128 // dt.itemsize, waves, wm, wn, 16, 1, 8, 0, 0, 0, split, 0, stages)
+
+
+def _fn(tb):
+    return (lambda x, w, b: tj.linear(x, w, b)) if tb else (lambda x, w, b: tj.matmul(x, w) + b)
+
+
+def _program(m, n, k, tb, dt, lead=()):
+    types = [TensorType((*lead, m, k), dt), TensorType((n, k) if tb else (k, n), dt), TensorType((n,), dt)]
+    return C.lower(tj.trace(_fn(tb), types), "hip")
+
+
+@pytest.mark.parametrize("dt", [DType.bf16, DType.f16, DType.f32])
+@pytest.mark.parametrize("tb", [True, False])
+def test_ring_takes_whole_chunks_and_compiles(dt, tb):
+    vk = 16 // dt.itemsize
+    cfg = _ring(32, 64, 4, 2, 2, 4, 1, dt)
+    ok = lambda c, m, n, k: hb.config_ok(c, dt, _program(m, n, k, tb, dt).kernels[0].anchor)  # noqa: E731
+    assert ok(cfg, 33, 5 * vk, 3 * vk) and ok(cfg, 1, vk, vk)
+    assert not ok(cfg, 33, 40, 3 * vk + 1)                       # rows of K that start inside a chunk
+    assert ok(cfg, 33, 5 * vk + 1, 64) == tb                     # NN: rows of N too
+    split = _ring(32, 64, 4, 2, 2, 4, 3, dt)
+    tk = cfg.TK
+    assert ok(split, 33, 40, 3 * tk) and ok(split, 33, 40, 4 * tk + vk)     # parts of 2, 2 and 1 K tiles
+    assert not ok(split, 33, 40, 2 * tk)                         # a part without a K tile
+    assert not ok(split, 33, 40, 4 * tk)                         # 2, 2, 0
+    p = _program(100, 520, 1032, tb, dt)
+    for c in (cfg, split):
+        src, launches = hb.generate(p, {0: c})
+        assert ("split_ws" in launches[0].meta) == (c.KSPLIT > 1)
+        hb.compile_source(src, "gfx950")
+
+
+def test_ring_candidates_are_valid_and_bounded():
+    for m, n, k in [(1, 768, 768), (64, 4096, 4096), (257, 1000, 8192), (8192, 8192, 8192), (3, 16, 16)]:
+        mm = _program(m, n, k, True, DType.bf16).kernels[0].anchor
+        for c in ring_candidates(m, n, k, 1, 2):
+            assert c.KSPLIT == 1 or -(-m // c.TM) * -(-n // c.TN) * c.KSPLIT <= 1024
+            if hb.config_ok(c, DType.bf16, mm):
+                src, (launch,) = hb.generate(_program(m, n, k, True, DType.bf16), {0: c})
+                assert launch.meta["lds_bytes"] <= 160 * 1024 and launch.grid[2] == c.KSPLIT
+
+
+def test_split_launches_share_the_workspace():
+    """Counters at the head of the block, as many as any launch has; partials behind them."""
+    dt = DType.bf16
+    g = tj.trace(lambda x, w, v: tj.linear(tj.linear(x, w), v),
+                 [TensorType((64, 1024), dt), TensorType((2048, 1024), dt), TensorType((512, 2048), dt)])
+    p = C.lower(g, "hip")
+    _, launches = hb.generate(p, {0: _ring(64, 64, 4, 2, 2, 4, 2, dt), 1: _ring(32, 32, 4, 2, 2, 4, 4, dt)})
+    args = hb.launch_args(launches, [[], []], {})
+    from tensorjit.runtime import hip as rt
+    assert args[0] == [(rt.WORKSPACE, 0, 32 * 4), (rt.WORKSPACE, 256, 2 * 32 * 64 * 64 * 4)]
+    assert args[1] == [(rt.WORKSPACE, 0, 32 * 4), (rt.WORKSPACE, 256, 4 * 32 * 32 * 32 * 4)]
+
+
+DEV = "cuda:0"
+
+
+def _native(fn, args, cfg):
+    p = C.lower(tj.trace(fn, [C.tensor_type_of(a) for a in args]), "hip")
+    (k,) = p.kernels
+    if not hb.config_ok(cfg, hb.compute_dtype(k.anchor), k.anchor):
+        return None
+    from tensorjit.runtime import hip as rt
+    src, ls = hb.generate(p, {0: cfg})
+    refs = [[(rt.INPUT, j) for j in range(len(k.inputs))] + [(rt.OUTPUT, 0)]]
+    return rt.NativeHipProgram(0, hb.compile_source(src, hb.arch_of(0), target=hb.target_of(0)), [l.name for l in ls],
+                               [(l.grid, l.block, 0) for l in ls], hb.launch_args(ls, refs, {}), 0, len(args), 1)
+
+
+def _integers(m, n, k, tb, dt, lead=(), seed=0):
+    """Operands in {-2..2}: every product and sum is exact in any order (bf16 outputs round
+    the same exact value)."""
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    r = lambda *s: torch.randint(-2, 3, s, device=DEV, generator=gen).to(TORCH[dt])  # noqa: E731
+    a, b, bias = r(*lead, m, k), r(n, k) if tb else r(k, n), r(n)
+    ref = (torch.matmul(a.double(), b.double().t().contiguous() if tb else b.double()) + bias.double()).to(TORCH[dt])
+    return [a, b, bias], ref
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [DType.bf16, DType.f16, DType.f32])
+@pytest.mark.parametrize("tb", [True, False])
+def test_ring_gemm_is_exact_at_the_edges(dt, tb):
+    """M one past and one short of tiles, N of one and several chunks, K short of a K tile,
+    of the ring, and ragged; K splits with unequal parts.  Twice each: the split's counters
+    are back at zero."""
+    tiles = [(32, 32, 4, 2, 2, 4), *RING_TILES, (64, 64, 8, 2, 4, 4)]
+    for i, (m, n, k) in enumerate([(1, 16, 16), (33, 136, 72), (63, 64, 1032), (129, 520, 264)]):
+        args, ref = _integers(m, n, k, tb, dt, seed=i)
+        out = torch.empty_like(ref)
+        ran = 0
+        for tm, tn, waves, wm, wn, stages in tiles:
+            for split in (1, 3):
+                prog = _native(_fn(tb), args, _ring(tm, tn, waves, wm, wn, stages, split, dt))
+                for _ in range(2 if prog else 0):
+                    out.fill_(77)
+                    prog.run([t.data_ptr() for t in args], [out.data_ptr()], torch.cuda.current_stream().cuda_stream)
+                    assert torch.equal(out, ref), (m, n, k, tm, tn, waves, split)
+                    ran += 1
+        assert ran >= 2 * len(tiles)
+
+
+@pytest.mark.gpu
+def test_ring_gemm_batched_and_epilogue_operand():
+    """A batch of products with a shared weight, and the residual ``x + linear(x, w)``."""
+    dt = DType.bf16
+    args, ref = _integers(40, 72, 200, True, dt, lead=(3,))
+    out = torch.empty_like(ref)
+    for split in (1, 2):
+        prog = _native(_fn(True), args, _ring(32, 64, 4, 2, 2, 4, split, dt))
+        prog.run([t.data_ptr() for t in args], [out.data_ptr()], torch.cuda.current_stream().cuda_stream)
+        assert torch.equal(out, ref)
+    (x, w, _), _ = _integers(50, 96, 96, True, dt)
+    want = (x.double() + x.double() @ w.double().t().contiguous()).to(torch.bfloat16)
+    out = torch.empty_like(want)
+    prog = _native(lambda x, w: x + tj.linear(x, w), [x, w], _ring(32, 32, 4, 2, 2, 4, 1, dt))
+    prog.run([x.data_ptr(), w.data_ptr()], [out.data_ptr()], torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+def test_split_products_on_several_streams_and_in_captured_graphs():
+    """One split program on three streams without any ordering between them, then captured on
+    a side stream and replayed with eager calls and synchronisation in between: the streams'
+    partials and counters are their own."""
+    dt = DType.bf16
+    fn = tj.jit(lambda x, w, b: tj.linear(x, w, b), tune=False)
+    cases = [_integers(48, 512, 6144, True, dt, seed=s) for s in range(3)]
+    cp = fn.compiled(*cases[0][0])
+    assert cp.matmul_configs[0].STAGES and cp.matmul_configs[0].KSPLIT > 1
+    streams = [torch.cuda.Stream() for _ in cases]
+    torch.cuda.synchronize()
+    got = [[] for _ in cases]
+    for _ in range(20):
+        for s, (args, _), g in zip(streams, cases, got):
+            with torch.cuda.stream(s):
+                g.append(fn(*args))
+    torch.cuda.synchronize()
+    for (_, ref), outs in zip(cases, got):
+        assert all(torch.equal(o, ref) for o in outs)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        a, b = fn(*cases[0][0]), fn(*cases[1][0])
+    for _ in range(3):
+        a.zero_(), b.zero_()
+        graph.replay()
+        eager = fn(*cases[2][0])
+        torch.cuda.synchronize()
+        assert torch.equal(a, cases[0][1]) and torch.equal(b, cases[1][1]) and torch.equal(eager, cases[2][1])
