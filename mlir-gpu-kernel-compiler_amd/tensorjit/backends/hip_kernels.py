@@ -168,13 +168,15 @@ def _nt_loads(streamed_input_bytes: int) -> bool:
     return streamed_input_bytes > MALL_BYTES
 
 
-def _load_lines(src: str, ctype_ptr: str, off: str, inner: int, vec: int, dst: str, nt: bool = False) -> list[str]:
+def _load_lines(src: str, ctype_ptr: str, off: str, inner: int, vec: int, dst: str, nt: bool = False,
+                unaligned: bool = False) -> list[str]:
     """Lines that fill ``dst[0..vec)`` with fp32 values of one vector of input ``src``
-    (``nt``: a contiguous vector load with the nontemporal hint)."""
+    (``nt``: a contiguous vector load with the nontemporal hint; ``unaligned``: one that may
+    start at any element)."""
     if vec == 1:
         return [f"{dst}[0] = tj_ld({src}_p[{off}]);"]
     if inner == 1:
-        return [f"tj_ldv{'_nt' if nt else ''}({src}_p + ({off}), {dst});"]
+        return [f"tj_ldv{'_u' if unaligned else ''}{'_nt' if nt else ''}({src}_p + ({off}), {dst});"]
     if inner == 0:
         return [f"{{ const float s_ = tj_ld({src}_p[{off}]);",
                 f"  for (int j = 0; j < {vec}; ++j) {dst}[j] = s_; }}"]
@@ -204,12 +206,28 @@ def gen_pointwise(g: KernelGen, nodes: list[Node], iter_shape: tuple[int, ...]) 
     # depends on the element count alone ([16384, 4095] fp32: 16-byte vectors, not scalars)
     flat = all(_flat_access(iter_shape, st) for st in in_st.values())
     row_len = numel if flat else (iter_shape[-1] if iter_shape else 1)
-    vec = _vec_for(row_len, numel, _kernel_dtype(k))
-    nvec = numel // vec
+    dt = _kernel_dtype(k)
+    vec = _vec_for(row_len, numel, dt)
+    # Rows of no whole number of vectors: every row gets ceil(len / vec) of them at unaligned
+    # addresses, the last one moved back to end with the row.  The elements it shares with its
+    # neighbour are computed twice, from the same inputs to the same bits.  One element per lane
+    # was bound by the count of its loads: the two-input gelu / sigmoid chain with row-broadcast
+    # scale and shift (one box, us) bf16 [16384, 4095] 150.7 -> 68.7 (5.9 TB/s), [50000, 301]
+    # 27.3 -> 17.4, fp32 [16384, 4095] 172.3 -> 131.5.
+    ragged = vec == 1 and vec_width(dt) <= row_len and row_len * 2 > vec_width(dt) and iter_shape != ()
+    if ragged:
+        vec = vec_width(dt)
+        vpr = -(-row_len // vec)
+        nvec = numel // row_len * vpr
+    else:
+        nvec = numel // vec
+    u_ = "_u" if ragged else ""
     unroll = POINTWISE_UNROLL
     per_block = POINTWISE_THREADS * unroll
     grid = max(1, -(-nvec // per_block))
-    idx_t = _index_type(numel)
+    idx_t = _index_type(nvec * vec)
+    e_of_vi = (f"vi / {vpr}u * {row_len}u + (vi % {vpr}u * {vec}u < {row_len - vec}u ? vi % {vpr}u * {vec}u : {row_len - vec}u)"
+               if ragged else f"vi * {vec}u")
     guard = nvec % per_block != 0
     inside = {id(n) for n in nodes}
     streamed = {id(n) for n in k.inputs if _streamed(iter_shape, in_st[id(n)])}
@@ -225,13 +243,13 @@ def gen_pointwise(g: KernelGen, nodes: list[Node], iter_shape: tuple[int, ...]) 
     L.append(f"    const {idx_t} vi = vbase + u * {POINTWISE_THREADS}u;")
     if guard:
         L.append(f"    if (vi >= {nvec}u) break;")
-    L.append(f"    const {idx_t} e = vi * {vec}u;")
+    L.append(f"    const {idx_t} e = {e_of_vi};")
     for n in k.inputs:
         st = in_st[id(n)]
         nm = g.names[id(n)]
         L += ["    " + s for s in _load_lines(nm, CTYPE[n.dtype], offset_expr("e", iter_shape, st),
                                              inner_stride(iter_shape, st), vec, f"{nm}_v[u]",
-                                             nt and id(n) in streamed)]
+                                             nt and id(n) in streamed, ragged)]
     L.append("  }")
     # phase 2: compute and store
     L.append("#pragma unroll")
@@ -239,7 +257,7 @@ def gen_pointwise(g: KernelGen, nodes: list[Node], iter_shape: tuple[int, ...]) 
     L.append(f"    const {idx_t} vi = vbase + u * {POINTWISE_THREADS}u;")
     if guard:
         L.append(f"    if (vi >= {nvec}u) break;")
-    L.append(f"    const {idx_t} e = vi * {vec}u;")
+    L.append(f"    const {idx_t} e = {e_of_vi};")
     for j, o in enumerate(k.outputs):
         L.append(f"    float o{j}_v[{vec}];")
     L.append("#pragma unroll")
@@ -261,10 +279,12 @@ def gen_pointwise(g: KernelGen, nodes: list[Node], iter_shape: tuple[int, ...]) 
         if vec == 1:
             L.append(f"    tj_st(out{j}_p + e, o{j}_v[0]);")
         else:
-            L.append(f"    tj_stv(out{j}_p + e, o{j}_v);")
+            L.append(f"    tj_stv{u_}(out{j}_p + e, o{j}_v);")
     L.append("  }")
     L.append("}")
-    meta = {"family": "pointwise", "vec": vec, "unroll": unroll, "numel": numel}
+    # "vec": elements per aligned vector; "unaligned": per unaligned one
+    meta = {"family": "pointwise", "vec": 1 if ragged else vec, "unaligned": vec if ragged else 0, "unroll": unroll,
+            "numel": numel}
     return "\n".join(L), Launch(g.fname, (grid, 1, 1), (POINTWISE_THREADS, 1, 1), 0, meta)
 
 
@@ -408,6 +428,17 @@ def gen_copy(g: KernelGen) -> tuple[str, Launch]:
 ROW_MAX_FLOATS = 32
 
 
+def late_floats(lanes: int, ragged: bool) -> int:
+    """Most values per lane that a row kernel's preloaded inputs may hold together; past it, a
+    gain or bias is loaded in the stage that reads it.  LayerNorm with gain and bias, one box,
+    us, all preloaded -> gain and bias late: 336 values bf16 [1856, 27691] 61.4 -> 42.9, fp16
+    [5256, 25536] 128.3 -> 85.4; 96 values on 1024 lanes (128 VGPRs each) fp32 [4096, 32768]
+    191.9 -> 181.5, and with a ragged row's masks bf16 [21409, 6269] 115.5 -> 93.2; but 96
+    values on up to 512 lanes fp32 [4096, 16384] 75.9 -> 81.3, bf16 [16384, 8192] 73.9 -> 75.7,
+    and 84 with masks fp32 [21409, 6269] 208.1 -> 214.2."""
+    return 64 if lanes > 512 else 90 if ragged else 128
+
+
 def row_geometry(N: int, vec: int, streaming_ok: bool) -> tuple[int, int, bool]:
     """(threads T, chunks per lane NCH, streaming).  Up to 256 lanes x 16 chunks of
     ``vec`` elements (rows with several stages: 512 lanes from 12 chunks at 256); then a
@@ -539,6 +570,15 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
 
     dt = _kernel_dtype(k)
     vec = _vec_for(N, N, dt)
+    # Rows of no whole number of vectors: unaligned 16-byte accesses, the row's last chunk moved
+    # back to end with the row; its first ``s0`` elements belong to the chunk before it (computed
+    # twice to the same bits, counted once by a sum).  Against one element per lane (one box, us):
+    # softmax bf16 [21409, 6269] 129.8 -> 89.5, LayerNorm 173.7 -> 92.9, RMSNorm fp32
+    # [16384, 4095] 97.5 -> 74.7 (7.2 TB/s), LayerNorm bf16 [50000, 301] 51.0 -> 15.0.
+    ragged = vec == 1 and N >= vec_width(dt)
+    if ragged:
+        vec = vec_width(dt)
+    u_ = "_u" if ragged else ""
     inside = {id(n) for n in k.nodes}
     escaping = {id(o): j for j, o in enumerate(k.outputs)}
     stage_of = {id(n): si for si, st in enumerate(stages) for n in st.nodes}
@@ -625,31 +665,42 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
         out = [f"  {{ const unsigned int n0 = ({c} * {T}u + tid) * {vec}u;"]
         if not full:
             out.append(f"  if (n0 < {N}u) {{")
+        if ragged:
+            out.append(f"  const unsigned int s0 = n0 + {vec}u > {N}u ? n0 + {vec}u - {N}u : 0u, nb = n0 - s0;")
         return out
+
+    nb = "nb" if ragged else "n0"
 
     def chunk_close() -> list[str]:
         return ["  }"] + ([] if full else ["  }"])
 
     def ext_load(n: Node, strides, dst: str) -> list[str]:
-        off = offset_expr(f"(r * {N}u + n0)", vec_shape, strides)
+        off = offset_expr(f"(r * {N}u + {nb})", vec_shape, strides)
         return _load_lines(g.names[id(n)], CTYPE[n.dtype], off, inner_stride(vec_shape, strides), vec, dst,
-                           nt and id(n) in ext_streamed)
+                           nt and id(n) in ext_streamed, ragged)
 
-    # register arrays: preloaded external inputs and kept values
+    # register arrays: preloaded external inputs and kept values.  A gain or bias (broadcast
+    # over rows, so cached) is loaded where its stage reads it instead when the arrays would
+    # hold too many values per lane.
+    readers = {i: sum(any(n in m.inputs for m in st.nodes) for st in stages) for i, (n, _) in vec_ext.items()}
+    late = {i for i in vec_ext if i not in ext_streamed and readers[i] == 1}
+    if NCH * vec * len(vec_ext) <= late_floats(T, ragged) or streaming or split:
+        late = set()
+    preloaded = {} if streaming else {i: v for i, v in vec_ext.items() if i not in late}
     preload = not streaming
     if preload:
-        for n, strides in vec_ext.values():
+        for n, strides in preloaded.values():
             nm = g.names[id(n)]
             L.append(f"  float {nm}_r[{NCH}][{vec}];")
         for n in kept:
             # lanes past the row's end never write theirs: start them at zero
             L.append(f"  float {g.names[id(n)]}_r[{NCH}][{vec}]{'' if full else ' = {}'};")
     preload_lines = []
-    if preload and vec_ext:
+    if preload and preloaded:
         preload_lines.append("#pragma unroll")
         preload_lines.append(f"  for (int c = 0; c < {NCH}; ++c) {{")
         preload_lines += ["  " + s for s in chunk_open("c")]
-        for n, strides in vec_ext.values():
+        for n, strides in preloaded.values():
             preload_lines += ["      " + s for s in ext_load(n, strides, f"{g.names[id(n)]}_r[c]")]
         preload_lines += ["  " + s for s in chunk_close()]
         preload_lines.append("  }")
@@ -659,7 +710,7 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
     def elem_value(n: Node) -> str:
         """fp32 value of input/earlier-stage node ``n`` at (chunk c, lane element j)."""
         if id(n) in vec_ext:
-            return f"{g.names[id(n)]}_r[c][j]" if preload else f"{g.names[id(n)]}_l[j]"
+            return f"{g.names[id(n)]}_r[c][j]" if id(n) in preloaded else f"{g.names[id(n)]}_l[j]"
         if id(n) in kept_ids:
             return f"{g.names[id(n)]}_r[c][j]"
         if id(n) in inside and not is_vec(n):
@@ -669,9 +720,9 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
     def elem_block(nodes: list[Node], inputs: list[Node], extra: list[str]) -> list[str]:
         """Per-element body for chunk c: loads (streaming), compute, stores, keeps."""
         out = []
-        if not preload:
+        if not preload or late:
             for n in inputs:
-                if id(n) in vec_ext:
+                if id(n) in vec_ext and id(n) not in preloaded:
                     out.append(f"float {g.names[id(n)]}_l[{vec}];")
                     out += ext_load(n, vec_ext[id(n)][1], f"{g.names[id(n)]}_l")
         stores = [n for n in nodes if id(n) in escaping and is_vec(n)]
@@ -692,8 +743,8 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
         out.append("}")
         for n in stores:
             j = escaping[id(n)]
-            dst = f"out{j}_p + r * {N}u + n0"
-            out.append(f"tj_stv({dst}, {g.names[id(n)]}_o);" if vec > 1 else f"tj_st({dst}, {g.names[id(n)]}_o[0]);")
+            dst = f"out{j}_p + r * {N}u + {nb}"
+            out.append(f"tj_stv{u_}({dst}, {g.names[id(n)]}_o);" if vec > 1 else f"tj_st({dst}, {g.names[id(n)]}_o[0]);")
         return out
 
     def chunk_loop(body: list[str]) -> list[str]:
@@ -752,7 +803,8 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
             is_max = red.op == "max"
             init = "(-__builtin_inff())" if is_max else "0.0f"
             xv = f"{g.names[id(x)]}_e" if x in prologue else elem_value(x)
-            upd = f"acc{st_i} = fmaxf(acc{st_i}, {xv});" if is_max else f"acc{st_i} += {xv};"
+            upd = (f"acc{st_i} = fmaxf(acc{st_i}, {xv});" if is_max else
+                   f"acc{st_i} += j >= (int)s0 ? {xv} : 0.0f;" if ragged else f"acc{st_i} += {xv};")
             L.append(f"  float acc{st_i} = {init};")
             used = [n for n in st.inputs if any(n in m.inputs for m in prologue + [red])]
             if split:
@@ -781,7 +833,7 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
             # per-row scalar stage over [rows] or [rows, 1]: linear index r addresses both
             L += scalar_lines(st.nodes, st, tuple(st.iter_shape), "r")
     L.append("}")
-    meta = {"family": "row", "vec": vec, "threads": T, "chunks": NCH, "streaming": streaming, "rows": nrows, "n": N,
+    meta = {"family": "row", "vec": vec, "unaligned": ragged, "threads": T, "chunks": NCH, "streaming": streaming, "rows": nrows, "n": N,
             "rows_per_block": R}
     if not split:
         return "\n".join(L), Launch(g.fname, (-(-nrows // R), 1, 1), (T * R, 1, 1), 0, meta)

@@ -81,24 +81,37 @@ template <typename T> __device__ __forceinline__ void tj_ldv(const T* p, float* 
 template <typename T> __device__ __forceinline__ void tj_ldv_nt(const T* p, float* v) {
   tj_unpackv(__builtin_nontemporal_load((const tj_u32x4*)p), p, v);
 }
-__device__ __forceinline__ void tj_stv(float* p, const float* v) {
+__device__ __forceinline__ tj_u32x4 tj_packv(const float*, const float* v) {
   tj_f32x4 x; x[0] = v[0]; x[1] = v[1]; x[2] = v[2]; x[3] = v[3];
-  tj_st16(p, __builtin_bit_cast(tj_u32x4, x));
+  return __builtin_bit_cast(tj_u32x4, x);
 }
-__device__ __forceinline__ void tj_stv(int* p, const float* v) {
+__device__ __forceinline__ tj_u32x4 tj_packv(const int*, const float* v) {
   tj_u32x4 x;
   for (int i = 0; i < 4; ++i) x[i] = (unsigned int)(int)v[i];
-  tj_st16(p, x);
+  return x;
 }
-__device__ __forceinline__ void tj_stv(unsigned short* p, const float* v) {
+__device__ __forceinline__ tj_u32x4 tj_packv(const unsigned short*, const float* v) {
   tj_u32x4 x;
   for (int i = 0; i < 4; ++i) x[i] = tj_f2bf2(v[2 * i], v[2 * i + 1]);
-  tj_st16(p, x);
+  return x;
 }
-__device__ __forceinline__ void tj_stv(_Float16* p, const float* v) {
+__device__ __forceinline__ tj_u32x4 tj_packv(const _Float16*, const float* v) {
   tj_u32x4 x;
   for (int i = 0; i < 4; ++i) x[i] = tj_f2h(v[2 * i]) | (tj_f2h(v[2 * i + 1]) << 16);
-  tj_st16(p, x);
+  return x;
+}
+template <typename T> __device__ __forceinline__ void tj_stv(T* p, const float* v) { tj_st16(p, tj_packv(p, v)); }
+// The same 16 bytes at any element's address (rows of an odd length): the global memory
+// instructions take unaligned addresses, and a wave's accesses stay contiguous.
+typedef tj_u32x4 tj_u32x4a2 __attribute__((aligned(2)));
+template <typename T> __device__ __forceinline__ void tj_ldv_u(const T* p, float* v) {
+  tj_unpackv(*(const tj_u32x4a2*)p, p, v);
+}
+template <typename T> __device__ __forceinline__ void tj_ldv_u_nt(const T* p, float* v) {
+  tj_unpackv(__builtin_nontemporal_load((const tj_u32x4a2*)p), p, v);
+}
+template <typename T> __device__ __forceinline__ void tj_stv_u(T* p, const float* v) {
+  __builtin_nontemporal_store(tj_packv(p, v), (tj_u32x4a2*)p);
 }
 
 // Fast fp32 math on the native transcendental units.  exp(x) = 2^(x*log2 e) on

@@ -1,0 +1,61 @@
+"""Rows of no whole number of 16-byte vectors (pointwise and row kernels) at the sizes where they can go wrong."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import tensorjit as tj
+from parity import close_f32, close_lowp
+from tensorjit import compiler as C
+from tensorjit.backends import hip_backend as hb
+from tensorjit.ir import DType, TensorType
+
+DEV = "cuda:0"
+DTYPES = [torch.float32, torch.bfloat16, torch.float16]
+
+
+def _close(out, ref, n=1):
+    if out.dtype == torch.float32:
+        close_f32(out, ref, scale=1e-5 * max(1.0, (n / 4096) ** 0.5))
+    else:
+        close_lowp(out, ref)
+
+
+def test_long_ragged_rows_compile():
+    def launch(fn, shapes, dt):
+        src, (l,) = hb.generate(C.lower(tj.trace(fn, [TensorType(s, dt) for s in shapes]), "hip"))
+        hb.compile_source(src, "gfx950")
+        return src, l
+
+    # three row arrays of 14 chunks: the gain and the bias are loaded in their stage
+    src, l = launch(lambda x, g, b: tj.layer_norm(x, g, b), [(64, 27691), (27691,), (27691,)], DType.bf16)
+    assert "in0_r[14][8]" in src and "in1_r[" not in src and "tj_stv_u" in src
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("rows,n", [(1, 9), (5, 17), (70, 1001), (3, 4097), (2, 12001), (2, 32767), (1, 300001), (33, 63)])
+def test_ragged_rows_match_float64(dt, rows, n):
+    """One element past and short of a vector, of a wave's chunks, of the 256 / 1024-lane
+    layouts, and a split reduction: sums count the last chunk's shared elements once."""
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    x = (torch.randn(rows, n, device=DEV, generator=gen) + 0.5).to(dt)
+    g = (1 + 0.1 * torch.randn(n, device=DEV, generator=gen)).to(dt)
+    X, G = x.double(), g.double()
+    _close(tj.jit(lambda a, b: tj.layer_norm(a, b, b))(x, g), F.layer_norm(X, (n,), G, G), n)
+    _close(tj.jit(lambda a: tj.softmax(a))(x), torch.softmax(X, -1), n)
+    _close(tj.jit(lambda a: tj.mean(a * a, axis=-1))(x), (X * X).mean(-1), n)
+    assert torch.equal(tj.jit(lambda a: tj.max(a, axis=-1))(x), x.amax(-1))
+    _close(tj.jit(lambda a, b: a * b + tj.sigmoid(b))(x, g), X * G + torch.sigmoid(G), 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [*DTYPES, torch.int32])
+@pytest.mark.parametrize("shape,other", [((4096, 33), (33,)), ((7, 9, 13), (9, 1)), ((5, 8, 9), (5, 1, 9)), ((1000, 1001), (1001,))])
+def test_ragged_pointwise_rows_are_exact(dt, shape, other):
+    """Row-broadcast, column-broadcast and middle-broadcast operands over odd rows: small
+    integers, every value exact; the last vector of a row overlaps its neighbour."""
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randint(-8, 9, shape, device=DEV, generator=gen).to(dt)
+    y = torch.randint(-8, 9, other, device=DEV, generator=gen).to(dt)
+    assert torch.equal(tj.jit(lambda a, b: a * b + a)(x, y), x * y + x)
+
