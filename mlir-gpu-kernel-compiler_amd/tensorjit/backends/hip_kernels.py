@@ -476,6 +476,13 @@ def row_geometry(N: int, vec: int, streaming_ok: bool) -> tuple[int, int, bool]:
 #   (two or more per lane lose 6-12%): RMSNorm bf16 [65536, 4096] 167 us against 173 us
 #   with 256 lanes x 2 chunks.
 # * longer rows: row_geometry (256 lanes x up to 16 chunks, then 1024 lanes).
+# Rows of up to 32 chunks (512 bytes) share a wave: 2-32 lanes each (the next power of two),
+# reduced inside their lanes; a wave for each left three lanes of four idle at 16 chunks.  One
+# box, us, one row per wave -> shared: softmax bf16 [185086, 64] 53.6 -> 7.8, fp32 [200000, 48]
+# 35.4 -> 11.4, [300000, 128] 54.3 -> 42.6, RMSNorm bf16 [262144, 128] 34.9 -> 19.2 (6.98 TB/s),
+# LayerNorm fp32 [50882, 48] 9.7 -> 8.5.  Few rows keep a wave each: the launch is all they cost.
+SHORT_ROW_MAX_CHUNKS = 32
+SHORT_ROW_MIN_ROWS = 1024
 WAVE_ROW_MAX_CHUNKS = 4
 WAVE_ROWS_PER_BLOCK = 4
 ONE_CHUNK_MAX_LANES = 1024
@@ -507,6 +514,9 @@ def row_shape(N: int, vec: int, streaming_ok: bool, reductions: int = 1, whole_r
     chunks; ``reductions``: reduction stages in the row kernel; ``whole_row_inputs``: every
     input read per element is a whole [rows, N] tensor (none is broadcast over rows)."""
     nv = -(-N // vec)
+    if nv <= SHORT_ROW_MAX_CHUNKS and N > 1:
+        lanes = 1 << max(1, (nv - 1).bit_length())
+        return RowShape(lanes, 1, False, WAVE_ROWS_PER_BLOCK * 64 // lanes)
     if nv <= 64 * WAVE_ROW_MAX_CHUNKS:
         return RowShape(64, -(-nv // 64), False, WAVE_ROWS_PER_BLOCK)
     if nv <= ONE_CHUNK_MAX_LANES:
@@ -630,11 +640,13 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
     else:
         shape = row_shape(N, vec, streaming_ok=len(stages) == 1, reductions=nred,
                           whole_row_inputs=len(ext_streamed) == len(vec_ext))
+        if shape.lanes < 64 and nrows < SHORT_ROW_MIN_ROWS:
+            shape = RowShape(64, 1, False, WAVE_ROWS_PER_BLOCK)
         T, NCH, streaming, R = shape.lanes, shape.chunks, shape.streaming, shape.rows_per_block
     if R > 1 and nrows < R * 256:
-        # too few rows to fill the chip with R-row workgroups: one row per workgroup
-        R = 1
-    nwaves = T // 64
+        # too few rows to fill the chip with 4-wave workgroups: one wave per workgroup
+        R = max(1, 64 // T)
+    nwaves = max(1, T // 64)
     # every chunk in bounds: whole rows of chunks, and with a split whole segments
     full = N % (T * vec * (NCH if split else 1)) == 0
 
@@ -651,10 +663,10 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
         L.append(f"  const {idx_t} r = blockIdx.x;")
         L.append("  const unsigned int tid = threadIdx.x;")
     else:
-        # one wave per row: reductions never leave the wave, so a wave past the last
-        # row simply returns
-        L.append(f"  const {idx_t} r = ({idx_t})blockIdx.x * {R}u + (threadIdx.x >> 6);")
-        L.append("  const unsigned int tid = threadIdx.x & 63u;")
+        # one wave, or a group of lanes of one, per row: reductions never leave it, so the
+        # lanes past the last row simply return
+        L.append(f"  const {idx_t} r = ({idx_t})blockIdx.x * {R}u + (threadIdx.x >> {T.bit_length() - 1});")
+        L.append(f"  const unsigned int tid = threadIdx.x & {T - 1}u;")
         if nrows % R:
             L.append(f"  if (r >= {nrows}u) return;")
     if scalars:
@@ -814,7 +826,7 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
                 L.append("  }")
             else:
                 L += chunk_loop(elem_block(prologue, used, [upd]))
-            L += _block_reduce_lines(f"acc{st_i}", is_max, nwaves, red_slot)
+            L += _block_reduce_lines(f"acc{st_i}", is_max, nwaves, red_slot, T)
             red_slot += 1
             if split:
                 # the partial of segments sb, sb + S, ...; the combine launch finishes the row
@@ -869,9 +881,12 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
 COMBINE_THREADS = 256
 
 
-def _block_reduce_lines(acc: str, is_max: bool, nwaves: int, slot: int) -> list[str]:
+def _block_reduce_lines(acc: str, is_max: bool, nwaves: int, slot: int, lanes: int = 64) -> list[str]:
     """All-reduce of ``acc`` over the workgroup: wave64 DPP, then (several waves) one
-    exchange through LDS slots ``tj_red[slot]`` behind one barrier."""
+    exchange through LDS slots ``tj_red[slot]`` behind one barrier; over a group of
+    ``lanes`` < 64 lanes, DPP alone."""
+    if lanes < 64:
+        return [f"  {acc} = tj_group_{'max' if is_max else 'sum'}<{lanes}>({acc});"]
     out = [f"  {acc} = {'tj_wave_max' if is_max else 'tj_wave_sum'}({acc});"]
     if nwaves > 1:
         out.append(f"  if ((tid & 63u) == 0u) tj_red[{slot}][tid >> 6] = {acc};")

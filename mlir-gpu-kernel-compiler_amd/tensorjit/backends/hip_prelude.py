@@ -167,6 +167,34 @@ __device__ __forceinline__ float tj_wave_max(float v) {
   return fmaxf(fmaxf(tj_lane(v, 0), tj_lane(v, 16)), fmaxf(tj_lane(v, 32), tj_lane(v, 48)));
 }
 
+// the same inside groups of L lanes (2-32, aligned; a group's lanes are all active): several
+// short rows per wave.  32 lanes: the two 16-lane rows' totals are exchanged by
+// v_permlane16_swap.
+template <int L> __device__ __forceinline__ float tj_group_sum(float v) {
+  if (L >= 2) v += TJ_DPP(v, 0xb1);
+  if (L >= 4) v += TJ_DPP(v, 0x4e);
+  if (L >= 8) v += TJ_DPP(v, 0x141);
+  if (L >= 16) v += TJ_DPP(v, 0x140);
+  if (L >= 32) {
+    const unsigned int u = __builtin_bit_cast(unsigned int, v);
+    const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    v = __builtin_bit_cast(float, (unsigned int)s[0]) + __builtin_bit_cast(float, (unsigned int)s[1]);
+  }
+  return v;
+}
+template <int L> __device__ __forceinline__ float tj_group_max(float v) {
+  if (L >= 2) v = fmaxf(v, TJ_DPP(v, 0xb1));
+  if (L >= 4) v = fmaxf(v, TJ_DPP(v, 0x4e));
+  if (L >= 8) v = fmaxf(v, TJ_DPP(v, 0x141));
+  if (L >= 16) v = fmaxf(v, TJ_DPP(v, 0x140));
+  if (L >= 32) {
+    const unsigned int u = __builtin_bit_cast(unsigned int, v);
+    const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    v = fmaxf(__builtin_bit_cast(float, (unsigned int)s[0]), __builtin_bit_cast(float, (unsigned int)s[1]));
+  }
+  return v;
+}
+
 // lane l and lane l ^ 32 combined: gfx950's v_permlane32_swap exchanges the two halves
 // of the wave in one VALU instruction (the attention kernel's query halves)
 __device__ __forceinline__ float tj_pair_max(float x) {

@@ -1,4 +1,5 @@
-"""Rows of no whole number of 16-byte vectors (pointwise and row kernels) at the sizes where they can go wrong."""
+"""Rows of no whole number of 16-byte vectors (pointwise and row kernels) and several short
+rows per wave, at the sizes where they can go wrong."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -20,12 +21,20 @@ def _close(out, ref, n=1):
         close_lowp(out, ref)
 
 
-def test_long_ragged_rows_compile():
+def test_short_rows_share_a_wave_and_long_ragged_rows_compile():
     def launch(fn, shapes, dt):
         src, (l,) = hb.generate(C.lower(tj.trace(fn, [TensorType(s, dt) for s in shapes]), "hip"))
         hb.compile_source(src, "gfx950")
         return src, l
 
+    for n, lanes in [(8, 2), (64, 8), (72, 16), (256, 32)]:
+        src, l = launch(tj.softmax, [(100000, n)], DType.bf16)
+        rows = 256 // lanes
+        assert l.grid == (-(-100000 // rows), 1, 1) and l.block == (256, 1, 1) and f"tj_group_sum<{lanes}>" in src
+    _, l = launch(tj.softmax, [(1024, 64)], DType.bf16)
+    assert l.grid == (128, 1, 1) and l.block == (64, 1, 1)           # too few rows for 4 waves each
+    _, l = launch(tj.softmax, [(1023, 64)], DType.bf16)
+    assert l.grid == (1023, 1, 1) and l.block == (64, 1, 1)          # fewer still: a wave per row
     # three row arrays of 14 chunks: the gain and the bias are loaded in their stage
     src, l = launch(lambda x, g, b: tj.layer_norm(x, g, b), [(64, 27691), (27691,), (27691,)], DType.bf16)
     assert "in0_r[14][8]" in src and "in1_r[" not in src and "tj_stv_u" in src
@@ -59,3 +68,16 @@ def test_ragged_pointwise_rows_are_exact(dt, shape, other):
     y = torch.randint(-8, 9, other, device=DEV, generator=gen).to(dt)
     assert torch.equal(tj.jit(lambda a, b: a * b + a)(x, y), x * y + x)
 
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("rows,n", [(4097, 2), (1025, 8), (33000, 24), (2049, 33), (5000, 64), (70001, 72), (1030, 127), (9001, 256)])
+def test_short_rows_match_float64(dt, rows, n):
+    """2-32 lanes per row, rows that do not fill the last wave or workgroup, ragged ones."""
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    x = torch.randn(rows, n, device=DEV, generator=gen).to(dt)
+    g = (1 + 0.1 * torch.randn(n, device=DEV, generator=gen)).to(dt)
+    X, G = x.double(), g.double()
+    _close(tj.jit(lambda a: tj.softmax(a))(x), torch.softmax(X, -1))
+    _close(tj.jit(lambda a, b: tj.rms_norm(a, b))(x, g), X * torch.rsqrt((X * X).mean(-1, keepdim=True) + 1e-6) * G)
+    assert torch.equal(tj.jit(lambda a: tj.max(a, axis=-1))(x), x.amax(-1))
