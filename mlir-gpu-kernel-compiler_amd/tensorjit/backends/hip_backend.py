@@ -290,7 +290,9 @@ def fold_elementwise_into_gemm(program: Program) -> Program:
     return Program(program.graph, kernels, program.aliases) if changed else program
 
 
-COL_MIN_BYTES = 512       # a column block's row (64 lanes) must hold at least this many bytes
+# a column block's row (64 lanes) must hold at least this many bytes, unless the reduced axis
+# is the leading one: its narrow rows are contiguous with one another
+COL_MIN_BYTES = 512
 
 
 def fold_transpose_into_reduce(program: Program) -> Program:
@@ -303,7 +305,7 @@ def fold_transpose_into_reduce(program: Program) -> Program:
     transpose keeps every other axis in order (the source is then [A, Rd, B] with the
     reduced axis Rd in the middle, and the outputs' order is [A, B]), each reduction's
     prologue is elementwise on the transposed value alone, nothing but the reductions'
-    values and epilogues escape, and a row of B holds at least COL_MIN_BYTES bytes.  With
+    values and epilogues escape, and a row of B holds at least COL_MIN_BYTES bytes or A is 1.  With
     one reduction, an elementwise kernel whose only output is the transposed source, read
     by nothing else, becomes its prologue too.  ``TENSORJIT_HIP_COLREDUCE=0`` keeps the
     reference plan."""
@@ -343,7 +345,7 @@ def _col_fold(kernels: list[Kernel], c: int, outs: set) -> tuple[dict[int, Kerne
     X = t.inputs[0]
     Sx = tuple(X.shape)
     A, Rd, B = math.prod(Sx[:a]), Sx[a], math.prod(Sx[a + 1:])
-    if B * X.dtype.itemsize < COL_MIN_BYTES:
+    if B * X.dtype.itemsize < COL_MIN_BYTES and A > 1:
         return None
     owner = {id(n): i for i, k in enumerate(kernels) for n in k.nodes}
     readers = sorted({owner.get(id(u), -1) for u in t.users})

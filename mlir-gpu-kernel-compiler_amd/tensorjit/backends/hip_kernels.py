@@ -966,6 +966,14 @@ def gen_colreduce(g: KernelGen) -> tuple[str, Launch | list[Launch]]:
     # inputs read per element of X: the folded elementwise kernel's inputs, or X itself
     xin = [n for n in k.inputs if n is X or any(n in m.inputs for m in xnodes)]
     xstr = {id(n): broadcast_strides(n.shape, Sx) for n in xin}
+    # rows of B that are no whole number of vectors: unaligned vectors, the last one moved back
+    # to end with the row (its columns beyond its neighbour's are reduced twice, to the same
+    # bits).  A vector must not cross a row of X's last dim unless every input is read flat.
+    # Sum over axis 0 (one box, us): fp32 [5896, 11382] 72.4 -> 44.8, bf16 [6357, 2813] 13.8 -> 10.7.
+    ragged = (vec == 1 and B >= vec_width(dt)
+              and (B == Sx[-1] or all(_flat_access(Sx, st) for st in xstr.values())))
+    if ragged:
+        vec = vec_width(dt)
     streamed = sum(math.prod(n.shape) * n.dtype.itemsize for n in xin if _streamed(Sx, xstr[id(n)]))
     nt = _nt_loads(streamed)
     nb, RS, S = col_layout(A, Rd, B, vec, streamed)
@@ -976,6 +984,10 @@ def gen_colreduce(g: KernelGen) -> tuple[str, Launch | list[Launch]]:
     init = "(-__builtin_inff())" if is_max else "0.0f"
     escaping = {id(o): j for j, o in enumerate(k.outputs)}
     nm = lambda n: g.names[id(n)]  # noqa: E731
+
+    narrow = A == 1 and B * dt.itemsize < COL_NARROW_BYTES
+    if narrow:
+        S, RS = col_narrow_layout(Rd, L, streamed)
 
     def fold(acc: str, v: str) -> str:
         return f"{acc} = fmaxf({acc}, {v});" if is_max else f"{acc} += {v};"
@@ -1002,6 +1014,28 @@ def gen_colreduce(g: KernelGen) -> tuple[str, Launch | list[Launch]]:
                 out.append(f"{ind}tj_st(out{escaping[id(n)]}_p + {r}, {nm(n)}_v);")
         return out
 
+    def element_lines(col: str, ind: str) -> list[str]:
+        """Fold row ``j``'s vector at column ``col`` into ``acc``."""
+        out = [f"{ind}const {idx_t} e = (({idx_t})ai * {Rd}u + j) * {B}u + {col};"]
+        for n in xin:
+            out.append(f"{ind}float {nm(n)}_l[{vec}];")
+            out += [ind + s for s in _load_lines(nm(n), CTYPE[n.dtype], offset_expr("e", Sx, xstr[id(n)]),
+                                                 inner_stride(Sx, xstr[id(n)]), vec, f"{nm(n)}_l",
+                                                 nt and _streamed(Sx, xstr[id(n)]), ragged)]
+        out += ["#pragma unroll", f"{ind}for (int q = 0; q < {vec}; ++q) {{"]
+        local = {id(n): f"{nm(n)}_l[q]" for n in xin}
+        for n in xnodes + tnodes:
+            out.append(f"{ind}  const float {nm(n)}_e = {emit_expr(n, local)};")
+            local[id(n)] = f"{nm(n)}_e"
+            if n is X:
+                local[id(t)] = local[id(X)]
+        if id(t) not in local:
+            local[id(t)] = local[id(X)]
+        return out + [f"{ind}  " + fold("acc[q]", local[id(red.inputs[0])]), f"{ind}}}"]
+
+    col_of = f"(lv * {vec}u < {B - vec}u ? lv * {vec}u : {B - vec}u)" if ragged else f"lv * {vec}u"
+    if narrow:
+        return _colreduce_narrow(g, Rd, B, vec, L, S, RS, idx_t, init, fold, element_lines, finish_lines, col_of)
     ws_param = ", float* __restrict__ ws_p" if S > 1 else ""
     C = [f'extern "C" __global__ __launch_bounds__({64 * COL_WAVES}) void {g.fname}({g.params()}{ws_param}) {{',
          f"  __shared__ float tj_col[{COL_WAVES}][{64 * vec}];",
@@ -1014,31 +1048,16 @@ def gen_colreduce(g: KernelGen) -> tuple[str, Launch | list[Launch]]:
          f"  for (int q = 0; q < {vec}; ++q) acc[q] = {init};",
          f"  if (lv < {L}u) {{",
          "#pragma unroll 4",
-         f"    for (unsigned int j = j0 + w; j < j1; j += {COL_WAVES}u) {{",
-         f"      const {idx_t} e = (({idx_t})ai * {Rd}u + j) * {B}u + lv * {vec}u;"]
-    for n in xin:
-        C.append(f"      float {nm(n)}_l[{vec}];")
-        C += ["      " + s for s in _load_lines(nm(n), CTYPE[n.dtype], offset_expr("e", Sx, xstr[id(n)]),
-                                                inner_stride(Sx, xstr[id(n)]), vec, f"{nm(n)}_l",
-                                                nt and _streamed(Sx, xstr[id(n)]))]
-    C += ["#pragma unroll", f"      for (int q = 0; q < {vec}; ++q) {{"]
-    local = {id(n): f"{nm(n)}_l[q]" for n in xin}
-    for n in xnodes + tnodes:
-        C.append(f"        const float {nm(n)}_e = {emit_expr(n, local)};")
-        local[id(n)] = f"{nm(n)}_e"
-        if n is X:
-            local[id(t)] = local[id(X)]
-    if id(t) not in local:
-        local[id(t)] = local[id(X)]
-    C.append("        " + fold("acc[q]", local[id(red.inputs[0])]))
-    C += ["      }", "    }", "  }"]
+         f"    for (unsigned int j = j0 + w; j < j1; j += {COL_WAVES}u) {{"]
+    C += element_lines(col_of, "      ")
+    C += ["    }", "  }"]
     # the 4 waves' partials through LDS, combined by wave 0 in a fixed order
     C += ["#pragma unroll", f"  for (int q = 0; q < {vec}; ++q) tj_col[w][lane * {vec}u + q] = acc[q];",
           "  __syncthreads();", f"  if (w != 0u || lv >= {L}u) return;",
           "#pragma unroll", f"  for (int q = 0; q < {vec}; ++q) {{", "    float a = tj_col[0][lane * %du + q];" % vec]
     for w in range(1, COL_WAVES):
         C.append("    " + fold("a", f"tj_col[{w}][lane * {vec}u + q]"))
-    C.append(f"    const {idx_t} r = ({idx_t})ai * {B}u + lv * {vec}u + q;")
+    C.append(f"    const {idx_t} r = ({idx_t})ai * {B}u + {col_of} + q;")
     if S == 1:
         C += finish_lines("r", "a", "    ")
     else:
@@ -1070,3 +1089,91 @@ def gen_colreduce(g: KernelGen) -> tuple[str, Launch | list[Launch]]:
     comb = Launch(g.fname + "_combine", (-(-AB // 64), 1, 1), (64 * CW, 1, 1), 0,
                   {"family": "colreduce_combine", "splits": S, "ws_arg": True, "outputs": AB})
     return "\n".join(C) + "\n\n" + "\n".join(D), [main, comb]
+
+
+# Rows of under 512 bytes, reduced over the leading axis: the 256 lanes of a workgroup hold as
+# many whole rows as fit (G of them, L vectors each), so its loads cover G * B consecutive
+# elements; the G partials of a column combine in a tree through LDS.  Split over S workgroups,
+# the last of them to finish folds the S partials (agent-coherent stores and loads, a counter in
+# the stream's workspace that is back at zero afterwards) and runs the finish: no second launch.
+# The plan's transpose and row reduction read and write the tensor twice more, and the transpose
+# of narrow rows gathers.  One box, us, plan -> here: bf16 [618418, 72] 1000 -> 24.3,
+# fp32 [177643, 30] 100 -> 10.4, [1000000, 16] 36.6 -> 17.2, bf16 [20000, 255] 31.2 -> 8.5,
+# [481, 26] 9.4 -> 7.2 (the host's share of a call).
+COL_NARROW_BYTES = 512
+COL_NARROW_LANES = 256
+
+
+def col_narrow_layout(Rd: int, L: int, streamed_bytes: int) -> tuple[int, int]:
+    """(workgroups S, rows per workgroup) of a narrow column reduction: four workgroups per CU
+    or fewer, four rows per lane group at least."""
+    G = COL_NARROW_LANES // L
+    forced = os.environ.get("TENSORJIT_HIP_COL_SPLITS")
+    if forced and forced.isdigit():
+        S = max(1, min(int(forced), Rd))
+    else:
+        # at most 16 partials per lane group for the finishing workgroup (bf16 [20000, 255], 8
+        # groups: 512 workgroups 61 us, 128 8.5)
+        S = max(1, min(col_workgroups_per_cu(streamed_bytes) * CU_COUNT, Rd // (4 * G), 16 * G, COL_MAX_SPLITS))
+    RS = -(-Rd // S)
+    return -(-Rd // RS), RS
+
+
+def _colreduce_narrow(g: KernelGen, Rd: int, B: int, vec: int, L: int, S: int, RS: int, idx_t: str, init: str, fold,
+                      element_lines, finish_lines, col_of: str) -> tuple[str, Launch]:
+    G, W = COL_NARROW_LANES // L, L * vec
+    part = W * 4
+    ws_param = ", unsigned int* cnt_p, float* ws_p" if S > 1 else ""
+
+    def tree() -> list[str]:
+        """acc of row groups 0 .. G-1 (threads (gi, lv), all at the barriers) into group 0's."""
+        out = ["#pragma unroll", f"  for (int q = 0; q < {vec}; ++q) if (gi < {G}u) tj_col[gi * {W}u + lv * {vec}u + q] = acc[q];",
+               "  __syncthreads();"]
+        n = G
+        while n > 1:
+            h = (n + 1) // 2
+            out += [f"  if (gi < {n - h}u) {{", "#pragma unroll", f"    for (int q = 0; q < {vec}; ++q) {{",
+                    "      " + fold("acc[q]", f"tj_col[(gi + {h}u) * {W}u + lv * {vec}u + q]"),
+                    f"      tj_col[gi * {W}u + lv * {vec}u + q] = acc[q];", "    }", "  }", "  __syncthreads();"]
+            n = h
+        return out
+
+    C = [f'extern "C" __global__ __launch_bounds__({COL_NARROW_LANES}) void {g.fname}({g.params()}{ws_param}) {{',
+         f"  __shared__ float tj_col[{G * W}];",
+         f"  const unsigned int tid = threadIdx.x, gi = tid / {L}u, lv = tid % {L}u, s = blockIdx.x, ai = 0u;",
+         f"  const unsigned int j0 = s * {RS}u, j1 = j0 + {RS}u < {Rd}u ? j0 + {RS}u : {Rd}u;",
+         f"  float acc[{vec}];", "#pragma unroll", f"  for (int q = 0; q < {vec}; ++q) acc[q] = {init};",
+         f"  if (gi < {G}u) {{", "#pragma unroll 8", f"    for (unsigned int j = j0 + gi; j < j1; j += {G}u) {{"]
+    C += element_lines(col_of, "      ") + ["    }", "  }"] + tree()
+    if S > 1:
+        # 16 bytes per access (a row's W floats are whole 16-byte chunks unless vec is 1)
+        off = f"{part}u + lv * {vec * 4}u"
+        if vec == 1:
+            st = [f"    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, acc[0]), rsW, (int)(s * {off}), 0, 16);"]
+            ld = ["      { " + fold("acc[0]", "__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsW, "
+                                     f"(int)(s2 * {off}), 0, 16))") + " }"]
+        else:
+            st, ld = [], []
+            for c in range(0, vec, 4):
+                st.append(f"    {{ tj_f32x4 p; p[0] = acc[{c}]; p[1] = acc[{c + 1}]; p[2] = acc[{c + 2}]; p[3] = acc[{c + 3}];"
+                          f" __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(tj_u32x4, p), rsW, (int)(s * {off} + {c * 4}u), 0, 16); }}")
+                ld.append(f"      {{ const tj_f32x4 p = __builtin_bit_cast(tj_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsW, (int)(s2 * {off} + {c * 4}u), 0, 16)); "
+                          + " ".join(fold(f"acc[{c + q}]", f"p[{q}]") for q in range(4)) + " }")
+        C += [f"  const __amdgpu_buffer_rsrc_t rsW = __builtin_amdgcn_make_buffer_rsrc((void*)ws_p, (short)0, {S * part}, 0x00020000);",
+              "  if (gi == 0u) {", *st, "  }",
+              "  __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): this wave's partial stores are done",
+              "  __shared__ unsigned int tj_last_;",
+              "  __syncthreads();",
+              f"  if (tid == 0u) tj_last_ = atomicAdd(cnt_p, 1u) == {S - 1}u ? 1u : 0u;",
+              "  __syncthreads();", "  if (tj_last_ == 0u) return;",
+              "#pragma unroll", f"  for (int q = 0; q < {vec}; ++q) acc[q] = {init};",
+              f"  if (gi < {G}u) {{", "#pragma unroll 8", f"    for (unsigned int s2 = gi; s2 < {S}u; s2 += {G}u) {{",
+              *ld, "    }", "  }",
+              *tree(), "  if (tid == 0u) *cnt_p = 0u;"]
+    C += ["  if (gi != 0u) return;", "#pragma unroll", f"  for (int q = 0; q < {vec}; ++q) {{", "    const float a = acc[q];",
+          f"    const {idx_t} r = {col_of} + q;"]
+    C += finish_lines("r", "a", "    ") + ["  }", "}"]
+    meta = {"family": "colreduce", "narrow": True, "vec": vec, "A": 1, "Rd": Rd, "B": B, "splits": S, "rows_per_wg": RS}
+    if S > 1:
+        meta["split_ws"] = (4, S * part)
+    return "\n".join(C), Launch(g.fname, (S, 1, 1), (COL_NARROW_LANES, 1, 1), 0, meta)
