@@ -354,6 +354,193 @@ def attention_splits(tiles: int, KB: int, pingpong: bool) -> int:
     return next((n for n in ok if tiles * n >= CU_COUNT), ok[-1])
 
 
+def few_queries(Sq: int) -> bool:
+    """At most 16 queries per head (decode steps): one 16-query MFMA column tile, keys dealt
+    to the waves.  The other schedules give every wave 32 query rows of its own, so three
+    waves of four repeat the first one's work there.  A forced
+    TENSORJIT_HIP_ATTENTION_WAVES keeps them."""
+    return Sq <= 16 and os.environ.get("TENSORJIT_HIP_ATTENTION_WAVES") not in ("4", "8")
+
+
+FEW_BLOCK = 32      # keys a wave takes at a time: one k step of the 16x16x32 PV MFMA
+
+
+def few_query_splits(batch: int, Sk: int, D: int, Dv: int) -> int:
+    """Key-range splits of the few-query kernel: the count of the least estimated time.  The
+    kernel takes its bytes at a rate that grows with the workgroups resident (two per CU, four
+    at head dims up to 64: their LDS tiles), or its steps of 128 keys one after the other;
+    splits add a combine launch.  Measured: 320 heads x 3000 keys x 128 89.5 us in one part, 77.7
+    in two, 75.4 in three (the fuller grid evens out the CUs); 512 heads x 4000 keys 152.8 in
+    one, 155.3 in two; 8 heads x 8192 keys 53.2 in one, 10.5 in 16.  Calls below
+    8 us are bound by the host's launch instead, which a second launch lengthens: 32 heads x
+    1500 keys x 64 8.5 us in one part, 10.5 in two."""
+    forced = os.environ.get("TENSORJIT_HIP_ATTENTION_SPLITS", "")
+    blocks = -(-Sk // FEW_BLOCK)
+    if forced.isdigit():
+        return max(1, min(int(forced), blocks))
+    slots = CU_COUNT * (2 if D + Dv > 128 else 4)
+    step_us = 0.55 + 0.27 * (D + Dv) / 256
+
+    def cost(n: int) -> float:
+        steps, groups = -(-(-(-blocks // n)) // 4), batch * n
+        resident = min(groups, slots)
+        rate = 7e6 * resident / (resident + 75)     # bytes per us: 5.7 TB/s at 320 workgroups
+        stream_us = groups * steps * 4 * FEW_BLOCK * (D + Dv) * 2 / rate
+        kernel_us = max(stream_us, -(-groups // slots) * steps * step_us) + (2.5 + 0.02 * n if n > 1 else 0.0)
+        return max(kernel_us, 7.7 if n == 1 else 10.2)
+
+    return min((n for n in range(1, 33) if n == 1 or blocks >= 4 * n), key=cost)
+
+
+def _gen_few_queries(fname: str, dt: DType, batch: int, Sq: int, Sk: int, D: int, Dv: int, scale: float,
+                     q: tuple[str, int], k: tuple[str, int], v: tuple[str, int], o: tuple[str, int]):
+    """Attention of at most 16 queries per head: bound by reading K and V once.
+
+    A workgroup of 4 waves owns one (batch, head), or one split of its keys.  Blocks of 32
+    keys are dealt to the waves round-robin, and each wave runs its own online softmax over
+    its blocks: no barrier until the end, when the four (reference, sum, output) triples are
+    combined through LDS.  A block goes memory -> registers -> the wave's own LDS tile, so
+    the loads are whole consecutive rows; the next block's 16 KiB (head dim 128) are in
+    flight while the present one is computed, and 8 waves per CU keep 128 KiB in flight,
+    twice what the memory latency needs.  The MFMAs are those of the 16x16x32 schedule:
+    ``S^T = K Q^T``, then ``O^T += V^T P^T`` with V^T by transposing LDS reads; 15 of 16
+    columns idle at one query, which leaves them under a tenth of the time.
+
+    Against the 4-wave schedule (us, before -> after, fp16 / bf16): 512 heads x 1 query x
+    4000 keys x 128 187.4 -> 154.1 (6.8 TB/s), 1024 heads x 1000 keys 125.0 -> 78.0, 768 x
+    2000 195 -> 116, 256 x 300 12.9 -> 7.7; 16 queries x 64 heads x 4096 keys x 64 18.5 ->
+    14.0.  Nontemporal loads past the last-level cache: 174 -> 153 at 512 x 4000.
+    """
+    from .hip_kernels import Launch, _nt_loads
+
+    (qoff, qst), (koff, kst), (voff, vst), (ooff, ost) = q, k, v, o
+    T = CTYPE[dt]
+    KB = -(-Sk // FEW_BLOCK)
+    NS = few_query_splits(batch, Sk, D, Dv)
+    KBL = -(-KB // NS)
+    NS = -(-KB // KBL)                          # every split has a block
+    idx_t = "unsigned long" if batch * max(Sq, Sk) * max(D, Dv) >= 2**31 else "unsigned int"
+    DP, VP = D + 8, Dv + 16     # row pitches: fragment and transposing reads meet no bank twice
+    opvec = "tj_bf16x8" if dt == DType.bf16 else "tj_f16x8"
+    mfma = "__builtin_amdgcn_mfma_f32_16x16x32_" + ("bf16" if dt == DType.bf16 else "f16")
+    cvt = "tj_f2bf2({0}, {1})" if dt == DType.bf16 else "tj_f2h({0}) | (tj_f2h({1}) << 16)"
+    cs = scale * 1.4426950408889634            # scores scaled into exp2's domain
+    ext, sign = ("fmaxf", "-") if cs > 0 else ("fminf", "")
+    masked = f"{sign}__builtin_inff()"
+    nt = _nt_loads(batch * Sk * (D + Dv) * dt.itemsize)
+    rd = "__builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) tj_i16x4*)"
+    lowest = "-3.402823466e+38f"     # a finite start: blocks of -inf scores only add zeros
+    fence = '__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier();'
+
+    def load(which: str, blk: str) -> list[str]:
+        reg, base, st, d = ("rk", "Kb", kst, D) if which == "k" else ("rv", "Vb", vst, Dv)
+        ptr = f"(const tj_u32x4*)&{base}[key * {st}u + (c % {d // 8}u) * 8u]"
+        out = ["#pragma unroll", f"for (int i = 0; i < {FEW_BLOCK * d // 512}; ++i) {{",
+               f"  const unsigned int c = i * 64u + lane;", f"  unsigned int key = ({blk}) * {FEW_BLOCK}u + c / {d // 8}u;"]
+        if Sk % FEW_BLOCK:
+            out.append(f"  key = key < {Sk}u ? key : {Sk - 1}u;")
+        return out + [f"  {reg}[i] = " + (f"__builtin_nontemporal_load({ptr});" if nt else f"*{ptr};"), "}"]
+
+    def store(which: str) -> list[str]:
+        reg, arr, d = ("rk", "Ks", D) if which == "k" else ("rv", "Vs", Dv)
+        return ["#pragma unroll", f"for (int i = 0; i < {FEW_BLOCK * d // 512}; ++i) {{",
+                f"  const unsigned int c = i * 64u + lane;",
+                f"  *(tj_u32x4*)&{arr}[wave][c / {d // 8}u][(c % {d // 8}u) * 8u] = {reg}[i];", "}"]
+
+    where = ([f"  const {idx_t} bh = blockIdx.x;", f"  const unsigned int b0 = 0u, b1 = {KB}u;"] if NS == 1 else
+             [f"  const {idx_t} bh = blockIdx.x / {NS}u;",
+              f"  const unsigned int sp = blockIdx.x % {NS}u, b0 = sp * {KBL}u, b1 = b0 + {KBL}u < {KB}u ? b0 + {KBL}u : {KB}u;"])
+    L = [f'extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) {fname}(',
+         f"    const {T}* __restrict__ in0_p, const {T}* __restrict__ in1_p, const {T}* __restrict__ in2_p,",
+         f"    {T}* __restrict__ out0_p{', float* __restrict__ ws_p' if NS > 1 else ''}) {{",
+         f"  __shared__ __attribute__((aligned(16))) {T} Ks[4][{FEW_BLOCK}][{DP}];",
+         f"  __shared__ __attribute__((aligned(16))) {T} Vs[4][{FEW_BLOCK}][{VP}];",
+         "  __shared__ float ml[4][16][2];",
+         "  const unsigned int tid = threadIdx.x, lane = tid % 64u, wave = __builtin_amdgcn_readfirstlane(tid / 64u);",
+         "  const unsigned int r16 = lane % 16u, g16 = lane / 16u;",
+         *where,
+         f"  const {T}* __restrict__ Qb = in0_p + ({qoff});",
+         f"  const {T}* __restrict__ Kb = in1_p + ({koff});",
+         f"  const {T}* __restrict__ Vb = in2_p + ({voff});",
+         f"  tj_u32x4 rk[{FEW_BLOCK * D // 512}], rv[{FEW_BLOCK * Dv // 512}];",
+         "  if (b0 + wave < b1) {", *("    " + x for x in load("k", "b0 + wave") + load("v", "b0 + wave")), "  }",
+         f"  {opvec} qf[{D // 32}];", f"  tj_f32x4 o[{Dv // 16}];",
+         f"  const unsigned int qr = r16 < {Sq}u ? r16 : {Sq - 1}u;",
+         "#pragma unroll", f"  for (int c = 0; c < {D // 32}; ++c) qf[c] = *(const {opvec}*)&Qb[qr * {qst}u + c * 32 + g16 * 8u];",
+         "#pragma unroll", f"  for (int u = 0; u < {Dv // 16}; ++u) o[u] = (tj_f32x4)(0.0f);",
+         f"  float m_run = {lowest}, l_run = 0.0f;",
+         "  for (unsigned int b = b0 + wave; b < b1; b += 4u) {",
+         *("    " + x for x in store("k") + store("v")),
+         "    if (b + 4u < b1) {", *("      " + x for x in load("k", "b + 4u") + load("v", "b + 4u")), "    }",
+         f"    {fence}",
+         "    tj_f32x4 s[2];",
+         "#pragma unroll", "    for (int t = 0; t < 2; ++t) {", "      s[t] = (tj_f32x4)(0.0f);",
+         "#pragma unroll", f"      for (int c = 0; c < {D // 32}; ++c)",
+         f"        s[t] = {mfma}(*(const {opvec}*)&Ks[wave][t * 16 + r16][c * 32 + g16 * 8u], qf[c], s[t], 0, 0, 0);", "    }",
+         f"    float mx = {masked};",
+         "#pragma unroll", "    for (int e = 0; e < 8; ++e) {"]
+    if Sk % FEW_BLOCK:
+        L.append(f"      if (b * {FEW_BLOCK}u + (e / 4) * 16u + g16 * 4u + e % 4 >= {Sk}u) s[e / 4][e % 4] = {masked};")
+    L += [f"      mx = {ext}(mx, s[e / 4][e % 4]);", "    }",
+          # lazy rescale, as in the other schedules: the reference moves only past 2^8
+          f"    const float mb = mx * {cs!r}f;",
+          "    if (__builtin_amdgcn_ballot_w64(mb > m_run + 8.0f)) {",
+          "      const float m_new = fmaxf(m_run, tj_quad_max(mb)), alpha = __builtin_amdgcn_exp2f(m_run - m_new);",
+          "      l_run *= alpha;",
+          "#pragma unroll", f"      for (int u = 0; u < {Dv // 16}; ++u) o[u] *= alpha;",
+          "      m_run = m_new;", "    }",
+          "    tj_u32x4 pw;",
+          "#pragma unroll", "    for (int w = 0; w < 4; ++w) {",
+          *(f"      const float e{h} = __builtin_amdgcn_exp2f(__builtin_fmaf(s[w / 2][2 * (w % 2) + {h}], {cs!r}f, -m_run));"
+            for h in range(2)),
+          "      l_run += e0 + e1;", f"      pw[w] = {cvt.format('e0', 'e1')};", "    }",
+          f"    const {opvec} pf = __builtin_bit_cast({opvec}, pw);",
+          "#pragma unroll", f"    for (int u = 0; u < {Dv // 16}; ++u) {{",
+          f"      const tj_i16x4 va = {rd}&Vs[wave][g16 * 4u + (lane % 16u) / 4u][u * 16 + (lane % 4u) * 4u]);",
+          f"      const tj_i16x4 vb = {rd}&Vs[wave][16u + g16 * 4u + (lane % 16u) / 4u][u * 16 + (lane % 4u) * 4u]);",
+          f"      o[u] = {mfma}(__builtin_bit_cast({opvec}, __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7)), pf, o[u], 0, 0, 0);",
+          "    }",
+          f"    {fence}",
+          "  }",
+          # the waves' results: rows [Sq][Dv] of each in its own V tile
+          "  const float l_wave = tj_quad_sum(l_run);",
+          "  if (g16 == 0u) { ml[wave][r16][0] = m_run; ml[wave][r16][1] = l_wave; }",
+          f"  if (r16 < {Sq}u) {{",
+          "#pragma unroll", f"    for (int u = 0; u < {Dv // 16}; ++u)",
+          f"      *(tj_f32x4*)((float*)&Vs[wave][0][0] + r16 * {Dv}u + u * 16 + g16 * 4u) = o[u];",
+          "  }",
+          "  __syncthreads();",
+          f"  for (unsigned int t = tid; t < {Sq * Dv // 4}u; t += 256u) {{",
+          f"    const unsigned int row = t / {Dv // 4}u, d4 = (t % {Dv // 4}u) * 4u;",
+          "    const float m = fmaxf(fmaxf(ml[0][row][0], ml[1][row][0]), fmaxf(ml[2][row][0], ml[3][row][0]));",
+          "    float l = 0.0f;", "    tj_f32x4 acc = (tj_f32x4)(0.0f);",
+          "#pragma unroll", "    for (int w = 0; w < 4; ++w) {",
+          "      const float f = __builtin_amdgcn_exp2f(ml[w][row][0] - m);",
+          "      l += f * ml[w][row][1];",
+          f"      acc += f * *(const tj_f32x4*)((const float*)&Vs[w][0][0] + row * {Dv}u + d4);", "    }"]
+    ml_base = NS * batch * Sq * Dv
+    if NS == 1:
+        L += [f"    {T}* __restrict__ Ob = out0_p + ({ooff});", "    const float inv = 1.0f / l;", "    tj_u32x2 pk;",
+              *(f"    pk[{i}] = {cvt.format(f'acc[{2 * i}] * inv', f'acc[{2 * i + 1}] * inv')};" for i in range(2)),
+              f"    *(tj_u32x2*)&Ob[row * {ost}u + d4] = pk;"]
+    else:
+        L += [f"    const unsigned int prow = (sp * {batch}u + (unsigned int)bh) * {Sq}u + row;",
+              f"    *(tj_f32x4*)&ws_p[prow * {Dv}u + d4] = acc;",
+              f"    if (d4 == 0u) {{ ws_p[{ml_base}u + prow * 2u] = m; ws_p[{ml_base}u + prow * 2u + 1u] = l; }}"]
+    L += ["  }", "}"]
+    meta = {"family": "attention", "dtype": dt.value, "batch": batch, "Sq": Sq, "Sk": Sk, "D": D, "Dv": Dv, "scale": scale,
+            "lds_bytes": 4 * FEW_BLOCK * (DP + VP) * 2 + 512, "flops": 2.0 * batch * Sq * Sk * (D + Dv), "splits": NS,
+            "schedule": "few-queries", "mfma": "16x16x32", "row_sums": "fp32"}
+    main = Launch(fname, (batch * NS, 1, 1), (256, 1, 1), 0, meta)
+    src = QUAD_HELPERS + "\n".join(L)
+    if NS == 1:
+        return src, main
+    meta["workspace"] = (ml_base + NS * batch * Sq * 2) * 4
+    meta["ws_arg"] = True
+    combine = gen_combine(fname, dt, batch, Sq, Dv, NS, ooff, ost, idx_t)
+    return src + "\n\n" + combine[0], [main, combine[1]]
+
+
 def _split_tile_lines(nq: int, batch: int, NS: int, KBL: int, idx_t: str) -> list[str]:
     """Workgroup -> (``bh``, ``qt``) and, with key splits, the split's first key block
     ``kb0``: the (batch*head, split) pairs are the XCD-grouped "heads" of ``_tile_lines``,
@@ -396,6 +583,10 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
 
     (qoff, qst), (koff, kst) = base_stride(layouts[0], Sq, D, q), base_stride(layouts[1], Sk, D, kk)
     (voff, vst), (ooff, ost) = base_stride(layouts[2], Sk, Dv, v), base_stride(out_layout, Sq, Dv, out)
+    if few_queries(Sq):
+        bdims = "x".join(str(d) for d in qb_dims) or "1"
+        return _gen_few_queries(f"tj{idx}_attention_{bdims}x{Sq}x{Sk}x{D}_{dt.value}_flash", dt, batch, Sq, Sk, D, Dv, scale,
+                                (qoff, qst), (koff, kst), (voff, vst), (ooff, ost))
     NW, QT = attention_layout(batch, Sq, D, Dv)
     assert QT == 1, "one query tile per wave"
     THREADS = NW * 64
@@ -1158,8 +1349,20 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
         return (QUAD_HELPERS if mi16 else "") + "\n".join(L), main
     meta["workspace"] = (ml_base + NS * batch * Sq * 2) * 4
     meta["ws_arg"] = True
-    # combine: one lane per 8 consecutive outputs of a row; weights 2^(m_s - max m) over
-    # the splits, out = sum_s w_s * O_s / sum_s w_s * l_s
+    combine = gen_combine(fname, dt, batch, Sq, Dv, NS, ooff, ost, idx_t)
+    return "\n".join(L) + "\n\n" + combine[0], [main, combine[1]]
+
+
+def gen_combine(fname: str, dt: DType, batch: int, Sq: int, Dv: int, NS: int, ooff: str, ost: int,
+                idx_t: str) -> tuple[str, "Launch"]:  # noqa: F821
+    """The second launch of a key-split attention: one lane per 8 consecutive outputs of a
+    row; weights 2^(m_s - max m) over the splits, out = sum_s w_s * O_s / sum_s w_s * l_s.
+    The workspace holds the partial rows [split][bh][Sq][Dv] and behind them the rows'
+    (running reference, sum) pairs [split][bh][Sq][2]."""
+    from .hip_kernels import Launch
+
+    T = CTYPE[dt]
+    ml_base = NS * batch * Sq * Dv
     runs = batch * Sq * (Dv // 8)
     cname = fname + "_combine"
     pack8 = ("tj_f2bf2({0}, {1})" if dt == DType.bf16 else "tj_f2h({0}) | (tj_f2h({1}) << 16)")
@@ -1199,4 +1402,4 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
          "}"]
     cmeta = {"family": "attention_combine", "splits": NS, "ws_arg": True, "batch": batch, "Sq": Sq, "Dv": Dv}
     comb = Launch(cname, (-(-runs // 256), 1, 1), (256, 1, 1), 0, cmeta)
-    return "\n".join(L) + "\n\n" + "\n".join(C), [main, comb]
+    return "\n".join(C), comb
