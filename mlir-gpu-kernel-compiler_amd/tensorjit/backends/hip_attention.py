@@ -337,21 +337,46 @@ def attention_layout(batch: int, Sq: int, D: int, Dv: int) -> tuple[int, int]:
 
 def attention_splits(tiles: int, KB: int, pingpong: bool) -> int:
     """Key-range splits per (batch*head, query tile) for grids that leave CUs idle: with
-    ``tiles`` workgroups short of one per CU, each workgroup takes an equal share of the
-    key blocks (``KB`` divisible by the split count, at least 2 blocks each) and writes
-    unnormalised partial outputs with their running maxima and sums; a second launch
-    combines them.  The smallest split count that reaches 256 workgroups, else the largest
-    one that divides ``KB``; 1 for the ping-pong schedule and for full grids.
-    TENSORJIT_HIP_ATTENTION_SPLITS=n forces n where it divides ``KB`` into >= 2-block parts."""
+    ``tiles`` workgroups short of one per CU, each workgroup takes a share of the ``KB`` key
+    blocks and writes unnormalised partial outputs with their running maxima and sums; a
+    second launch combines them.  Shares are equal with at least 2 blocks each, or differ by
+    one block with at least 3.  The smallest split count that reaches 256 workgroups, else the
+    largest; 1 for the ping-pong schedule and for full grids.  ``key_splits`` takes this many
+    or fewer.
+    TENSORJIT_HIP_ATTENTION_SPLITS=n forces n where every share has at least 2 blocks."""
     forced = os.environ.get("TENSORJIT_HIP_ATTENTION_SPLITS", "")
-    ok = [n for n in range(2, 33) if KB % n == 0 and KB // n >= 2]
     if pingpong:
         return 1
     if forced.isdigit():
-        return int(forced) if int(forced) in ok else 1
+        return int(forced) if 2 <= int(forced) <= 32 and KB // int(forced) >= 2 else 1
+    ok = _split_counts(KB)
     if tiles >= CU_COUNT or not ok:
         return 1
     return next((n for n in ok if tiles * n >= CU_COUNT), ok[-1])
+
+
+def _split_counts(KB: int) -> list[int]:
+    return [n for n in range(2, 33) if KB // n >= (2 if KB % n == 0 else 3)]
+
+
+def key_splits(tiles: int, KB: int, pingpong: bool, dims: int, out_elems: int) -> int:
+    """The split count of the least estimated time, for ``dims`` = D + Dv and ``out_elems``
+    outputs.  A CU's second workgroup takes as long as its first (2.85 against 1.27 us per key
+    block at head dim 128), so splits pay only by reaching idle CUs, and the fp32 partials
+    cost 2.7 us and 0.58 us per MB.  us in 1 / 2 / 3 / 4 parts (the estimate's choice first):
+    8 heads x 1100 x 128 3: 20.8 (25.7 / 22.1 / - / 27.3), 8 x 1850 x 64 2: 19.2 (21.7 / - /
+    22.4 / 21.8), 64 x 330 x 64 1: 7.9 (- / 15.3 / 18.9), 32 x 600 x 128 1: 19.4 (- / 26.9 /
+    23.8 / 28.8), 8 x 2600 x 128 1: 52.9 (- / 55.5 / 47.8 / 54.5)."""
+    most = attention_splits(tiles, KB, pingpong)
+    if most == 1 or os.environ.get("TENSORJIT_HIP_ATTENTION_SPLITS", "").isdigit():
+        return most
+
+    def cost(n: int) -> float:
+        kernel_us = 2.3 + -(-tiles * n // CU_COUNT) * -(-KB // n) * (0.23 + 1.04 * dims / 256)
+        # a call of one launch takes the host 7.7 us, of two 10.2
+        return max(7.7, kernel_us) if n == 1 else max(10.2, kernel_us + 2.7 + 0.58e-6 * out_elems * 4 * n)
+
+    return min([1] + [n for n in _split_counts(KB) if n <= most], key=cost)
 
 
 def few_queries(Sq: int) -> bool:
@@ -541,14 +566,19 @@ def _gen_few_queries(fname: str, dt: DType, batch: int, Sq: int, Sk: int, D: int
     return src + "\n\n" + combine[0], [main, combine[1]]
 
 
-def _split_tile_lines(nq: int, batch: int, NS: int, KBL: int, idx_t: str) -> list[str]:
-    """Workgroup -> (``bh``, ``qt``) and, with key splits, the split's first key block
-    ``kb0``: the (batch*head, split) pairs are the XCD-grouped "heads" of ``_tile_lines``,
-    so the query tiles that share a key range share an XCD's L2."""
+def _split_tile_lines(nq: int, batch: int, NS: int, KB: int, idx_t: str) -> list[str]:
+    """Workgroup -> (``bh``, ``qt``) and, with key splits, the split ``sp`` and its first key
+    block ``kb0``: the (batch*head, split) pairs are the XCD-grouped "heads" of
+    ``_tile_lines``, so the query tiles that share a key range share an XCD's L2.  Where
+    ``NS`` does not divide ``KB``, the first ``long`` splits have one block more."""
     if NS == 1:
         return _tile_lines(nq, batch, idx_t)
     lines = [x.replace(" bh = ", " vh = ") for x in _tile_lines(nq, batch * NS, idx_t)]
-    return lines + [f"  const {idx_t} bh = vh / {NS}u;", f"  const unsigned int kb0 = (unsigned int)(vh % {NS}u) * {KBL}u;"]
+    KBL = -(-KB // NS)
+    long = KB - NS * (KBL - 1)
+    kb0 = f"sp * {KBL}u" if long == NS else f"sp * {KBL}u - (sp > {long}u ? sp - {long}u : 0u)"
+    return lines + [f"  const {idx_t} bh = vh / {NS}u;",
+                    f"  const unsigned int sp = (unsigned int)(vh % {NS}u), kb0 = {kb0};"]
 
 
 def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
@@ -596,8 +626,10 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
     BQ = BQ_PER_WAVE * QT * NW
     KB = -(-Sk // BKV)
     nq = -(-Sq // BQ)
-    NS = attention_splits(batch * nq, KB, pingpong)
-    KBL = KB // NS                              # key blocks per workgroup
+    NS = key_splits(batch * nq, KB, pingpong, D + Dv, batch * Sq * Dv)
+    KBL = -(-KB // NS)                          # key blocks per workgroup
+    long = KB - NS * (KBL - 1)                  # splits of KBL blocks; the others have one less
+    uneven = long < NS
     kb0 = "" if NS == 1 else "kb0 + "           # the workgroup's first key block
     DP = D + 8                                  # 16-byte row padding: conflict-free fragment reads
     # V rows: a transposing read touches 8 rows x 64 bytes; a pitch of 32 or 96 (mod 128)
@@ -711,7 +743,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
          *lds_decl,
          "  const unsigned int tid = threadIdx.x, lane = tid % 64u, wave = tid / 64u;",
          "  const unsigned int g = lane / 32u, col = lane % 32u;",
-         *_split_tile_lines(nq, batch, NS, KBL, idx_t),
+         *_split_tile_lines(nq, batch, NS, KB, idx_t),
          f"  const {T}* __restrict__ Qb = in0_p + ({qoff});",
          f"  const {T}* __restrict__ Kb = in1_p + ({koff});",
          f"  const {T}* __restrict__ Vb = in2_p + ({voff});",
@@ -766,7 +798,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
         out_l = ["#pragma unroll", f"for (int i = 0; i < {KC}; ++i) {{",
                  f"  const unsigned int c = i * {THREADS}u + tid, row = c / {D // 8}u, d8 = (c % {D // 8}u) * 8u;",
                  f"  unsigned int key = ({kb0}{blk}) * {BKV}u + row;"]
-        if ragged:
+        if ragged or uneven:
             out_l.append(f"  key = key < {Sk}u ? key : {Sk - 1}u;")
         return out_l + [f"  rk[i] = *(const tj_u32x4*)&Kb[key * {kst}u + d8];", "}"]
 
@@ -774,7 +806,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
         out_l = ["#pragma unroll", f"for (int i = 0; i < {VC}; ++i) {{",
                  f"  const unsigned int c = i * {THREADS}u + tid, row = c / {Dv // 8}u, d8 = (c % {Dv // 8}u) * 8u;",
                  f"  unsigned int key = ({kb0}{blk}) * {BKV}u + row;"]
-        if ragged:
+        if ragged or uneven:
             out_l.append(f"  key = key < {Sk}u ? key : {Sk - 1}u;")
         return out_l + [f"  rv[i] = *(const tj_u32x4*)&Vb[key * {vst}u + d8];", "}"]
 
@@ -841,7 +873,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
         if mi16:
             return block_max16(sc, j, pre)
         mask = None
-        if ragged and j == KBL - 1:
+        if ragged and (j == KBL - 1 or uneven and j == KBL - 2):
             mask = f"{j * BKV}" if NS == 1 else f"(int)kb0 * {BKV} + {j * BKV}"
         elif ragged and j is None and pingpong:
             mask = "(int)jj"
@@ -962,7 +994,10 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
             out += ["    {"] + ["      " + x for x in iteration("j + 1u", None, 1, True, True, True, True, True)] + ["    }"]
             out.append("  }")
         for j in range(2 * npair, KBL):
-            out.append(f"  {{  // block {j}")
+            # shorter splits have loaded and scored a block of the next split (rows clamped to
+            # the last key behind the last split) and leave it out
+            guard = f"if (sp < {long}u) " if uneven and j == KBL - 1 else ""
+            out.append(f"  {guard}{{  // block {j}")
             out += ["    " + x for x in iteration(f"{j}u", j, j % 2, j + 1 < KBL, j + 2 < KBL, j + 1 < KBL, j + 3 < KBL,
                                                   j + 2 < KBL)]
             out.append("  }")
@@ -1314,7 +1349,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
                 "    const unsigned int qrow = qrow0 + q * 32u;",
                 "    const float l_tot = tj_pair_sum(l_run[q]);",
                 f"    if (qrow < {Sq}u) {{",
-                f"      const unsigned int prow = ((kb0 / {KBL}u) * {batch}u + (unsigned int)bh) * {Sq}u + qrow;",
+                f"      const unsigned int prow = (sp * {batch}u + (unsigned int)bh) * {Sq}u + qrow;",
                 "#pragma unroll",
                 f"      for (int u = 0; u < {Dv // 32}; ++u)",
                 "#pragma unroll",

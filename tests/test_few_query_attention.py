@@ -1,12 +1,14 @@
-"""Attention of at most 16 queries per head: edges of its key blocks, waves and splits."""
+"""Attention of few queries or few heads: edges of the key blocks, the waves and the key splits."""
 from __future__ import annotations
+
+import re
 
 import pytest
 import torch
 
 import tensorjit as tj
 from tensorjit.backends import hip_backend as hb
-from tensorjit.backends.hip_attention import few_query_splits, fuse_attention
+from tensorjit.backends.hip_attention import _split_tile_lines, few_query_splits, fuse_attention
 from tensorjit.compiler import lower
 from tensorjit.ir import DType, TensorType
 
@@ -24,7 +26,6 @@ def launches_of(shapes, dt=DType.bf16):
 @pytest.mark.parametrize("Sq,Sk,D,Dv", [(1, 1, 32, 32), (16, 4096, 96, 128), (4, 130, 64, 32)])
 def test_few_queries_compile_and_keep_in_their_buffers(Sq, Sk, D, Dv, dt):
     src, launches = launches_of([(3, Sq, D), (3, Sk, D), (3, Sk, Dv)], dt)
-    launches = launches if isinstance(launches, list) else [launches]
     m = launches[0].meta
     assert m["schedule"] == "few-queries" and launches[0].grid == (3 * m["splits"], 1, 1)
     assert len(launches) == (2 if m["splits"] > 1 else 1)
@@ -71,6 +72,48 @@ def test_few_queries_match_fp32_attention(shape, splits, scale, dt, monkeypatch)
     out = f(q, k, v)
     assert f.compiled(q, k, v).launches[0].meta["schedule"] == "few-queries"
     p = torch.softmax(torch.matmul(q.cpu().double(), k.cpu().double().transpose(-1, -2)) * scale, -1)
+    ref = torch.matmul(p, v.cpu().double())
+    eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    bound = eps * (torch.matmul(p, v.cpu().double().abs()) + ref.abs()) + 1e-6
+    assert bool(((out.cpu().double() - ref).abs() <= bound).all())
+
+
+def test_shares_of_the_key_blocks_cover_them():
+    """Key splits of the tiled schedule that do not divide the blocks: the emitted first blocks
+    and the guarded last one give every block to exactly one split."""
+    for KB in range(2, 70):
+        for n in (n for n in range(2, 33) if KB // n >= 2):
+            KBL = -(-KB // n)
+            lines = " ".join(_split_tile_lines(2, 3, n, KB, "unsigned int"))
+            expr = re.search(r"kb0 = (.*?);", lines).group(1)
+            m = re.fullmatch(r"sp \* (\d+)u(?: - \(sp > (\d+)u \? sp - \2u : 0u\))?", expr)
+            assert int(m.group(1)) == KBL
+            long = int(m.group(2)) if m.group(2) else n
+            seen = [sp * KBL - max(0, sp - long) + j for sp in range(n) for j in range(KBL if sp < long else KBL - 1)]
+            assert seen == list(range(KB)), (KB, n)
+
+
+@pytest.mark.parametrize("shapes,splits", [
+    ([(8, 1100, 128)] * 3, 3), ([(8, 1450, 128)] * 3, 2), ([(64, 330, 64)] * 3, 1), ([(32, 600, 128)] * 3, 1)])
+def test_key_splits_reach_idle_compute_units_only(shapes, splits):
+    assert launches_of(shapes)[1][0].meta["splits"] == splits
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,splits", [((2, 100, 300, 64, 64), "2"), ((3, 129, 448, 128, 128), "3"),
+                                          ((2, 40, 833, 64, 128), "4"), ((1, 260, 1025, 96, 32), "5")])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_uneven_key_splits_match_fp32_attention(shape, splits, dt, monkeypatch):
+    """5 blocks in 2 parts (ragged), 7 in 3, 14 in 4 (ragged), 17 in 5 (one key in the last block)."""
+    monkeypatch.setenv("TENSORJIT_HIP_ATTENTION_SPLITS", splits)
+    B, Sq, Sk, D, Dv = shape
+    gen = torch.Generator(device="cuda").manual_seed(Sk)
+    q, k, v = [torch.randn(B, n, d, device="cuda", generator=gen).to(dt) for n, d in ((Sq, D), (Sk, D), (Sk, Dv))]
+    print(f"uneven splits {shape} {splits} {dt}", flush=True)
+    f = tj.jit(attention(0.1))
+    out = f(q, k, v)
+    assert f.compiled(q, k, v).launches[0].meta["splits"] == int(splits)
+    p = torch.softmax(torch.matmul(q.cpu().double(), k.cpu().double().transpose(-1, -2)) * 0.1, -1)
     ref = torch.matmul(p, v.cpu().double())
     eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
     bound = eps * (torch.matmul(p, v.cpu().double().abs()) + ref.abs()) + 1e-6
