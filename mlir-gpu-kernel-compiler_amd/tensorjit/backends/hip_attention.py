@@ -83,13 +83,12 @@ __device__ __forceinline__ float tj_quad_max(float x) {
   const auto s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
   return tj_pair_max(fmaxf(__builtin_bit_cast(float, (unsigned int)s[0]), __builtin_bit_cast(float, (unsigned int)s[1])));
 }
-typedef _Float16 tj_f16x2q __attribute__((ext_vector_type(2)));
 // sum of the two 16-bit probabilities of a packed pair, added to acc (v_dot2c with ones)
 __device__ __forceinline__ float tj_pair_acc_bf16(unsigned int p, float acc) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(tj_bf16x2, p), __builtin_bit_cast(tj_bf16x2, 0x3F803F80u), acc, false);
 }
 __device__ __forceinline__ float tj_pair_acc_f16(unsigned int p, float acc) {
-  return __builtin_amdgcn_fdot2(__builtin_bit_cast(tj_f16x2q, p), __builtin_bit_cast(tj_f16x2q, 0x3C003C00u), acc, false);
+  return __builtin_amdgcn_fdot2(__builtin_bit_cast(tj_f16x2, p), __builtin_bit_cast(tj_f16x2, 0x3C003C00u), acc, false);
 }
 __device__ __forceinline__ float tj_quad_sum(float x) {
   const unsigned int u = __builtin_bit_cast(unsigned int, x);
@@ -448,7 +447,7 @@ def _gen_few_queries(fname: str, dt: DType, batch: int, Sq: int, Sk: int, D: int
     DP, VP = D + 8, Dv + 16     # row pitches: fragment and transposing reads meet no bank twice
     opvec = "tj_bf16x8" if dt == DType.bf16 else "tj_f16x8"
     mfma = "__builtin_amdgcn_mfma_f32_16x16x32_" + ("bf16" if dt == DType.bf16 else "f16")
-    cvt = "tj_f2bf2({0}, {1})" if dt == DType.bf16 else "tj_f2h({0}) | (tj_f2h({1}) << 16)"
+    cvt = "tj_f2bf2({0}, {1})" if dt == DType.bf16 else "tj_f2h2({0}, {1})"
     cs = scale * 1.4426950408889634            # scores scaled into exp2's domain
     ext, sign = ("fmaxf", "-") if cs > 0 else ("fminf", "")
     masked = f"{sign}__builtin_inff()"
@@ -649,8 +648,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
     if dt == DType.bf16:
         pack4 = "tj_f2bf2({0}, {1}) | ((unsigned long)tj_f2bf2({2}, {3}) << 32)"
     else:
-        pack4 = ("(unsigned long)(tj_f2h({0}) | (tj_f2h({1}) << 16)) | "
-                 "((unsigned long)(tj_f2h({2}) | (tj_f2h({3}) << 16)) << 32)")
+        pack4 = "tj_f2h2({0}, {1}) | ((unsigned long)tj_f2h2({2}, {3}) << 32)"
 
     # head dim 128, ping-pong: K and V blocks go straight from memory into LDS (DMA)
     dma = (pingpong and D == 128 and Dv == 128 and NS == 1
@@ -902,7 +900,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
 
     def probs(sc: str) -> list[str]:
         """exp2 of the block's scores, the running sums, and the P^T operands (chunk 2t+h)."""
-        cvt = ("tj_f2bf2({0}, {1})" if dt == DType.bf16 else "tj_f2h({0}) | (tj_f2h({1}) << 16)")
+        cvt = ("tj_f2bf2({0}, {1})" if dt == DType.bf16 else "tj_f2h2({0}, {1})")
         if mi16:
             return probs16(sc, cvt, not balanced)
         return ["#pragma unroll", f"for (int q = 0; q < {QT}; ++q) {{",
@@ -1400,7 +1398,7 @@ def gen_combine(fname: str, dt: DType, batch: int, Sq: int, Dv: int, NS: int, oo
     ml_base = NS * batch * Sq * Dv
     runs = batch * Sq * (Dv // 8)
     cname = fname + "_combine"
-    pack8 = ("tj_f2bf2({0}, {1})" if dt == DType.bf16 else "tj_f2h({0}) | (tj_f2h({1}) << 16)")
+    pack8 = ("tj_f2bf2({0}, {1})" if dt == DType.bf16 else "tj_f2h2({0}, {1})")
     C = [f'extern "C" __global__ void __launch_bounds__(256) {cname}(',
          f"    const {T}* __restrict__ in0_p, const {T}* __restrict__ in1_p, const {T}* __restrict__ in2_p,",
          f"    {T}* __restrict__ out0_p, const float* __restrict__ ws_p) {{",

@@ -81,3 +81,17 @@ def test_short_rows_match_float64(dt, rows, n):
     _close(tj.jit(lambda a: tj.softmax(a))(x), torch.softmax(X, -1))
     _close(tj.jit(lambda a, b: tj.rms_norm(a, b))(x, g), X * torch.rsqrt((X * X).mean(-1, keepdim=True) + 1e-6) * G)
     assert torch.equal(tj.jit(lambda a: tj.max(a, axis=-1))(x), x.amax(-1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [4096, 4099])
+def test_fp16_stores_round_to_nearest_even(n):
+    """Products of fp16 values rounded back to fp16: ties, subnormals, overflows to infinity and
+    NaN come out with torch's bits."""
+    bits = torch.arange(-(1 << 15), 1 << 15, device="cuda", dtype=torch.int32).to(torch.int16).view(torch.float16)
+    a = bits[torch.randperm(1 << 16, device="cuda")][:n * 15].reshape(15, n)
+    b = bits[torch.randperm(1 << 16, device="cuda")][:n * 15].reshape(15, n)
+    out, ref = tj.jit(lambda x, y: x * y)(a, b), (a.float() * b.float()).half()
+    nan = ref.isnan()
+    assert torch.equal(out.isnan(), nan)
+    assert torch.equal(out.view(torch.int16)[~nan], ref.view(torch.int16)[~nan])
