@@ -570,6 +570,9 @@ def row_split(nrows: int, N: int, vec: int, itemsize: int) -> RowSplit | None:
     return RowSplit(nch, segs, splits) if splits > 1 else None
 
 
+RAGGED_MIN_ROWS = 64
+
+
 def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[str, Launch]:
     k = g.k
     nrows = math.prod(rows) if rows else 1
@@ -585,7 +588,7 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
     # twice to the same bits, counted once by a sum).  Against one element per lane (one box, us):
     # softmax bf16 [21409, 6269] 129.8 -> 89.5, LayerNorm 173.7 -> 92.9, RMSNorm fp32
     # [16384, 4095] 97.5 -> 74.7 (7.2 TB/s), LayerNorm bf16 [50000, 301] 51.0 -> 15.0.
-    ragged = vec == 1 and N >= vec_width(dt)
+    ragged = vec == 1 and N >= vec_width(dt) and nrows >= RAGGED_MIN_ROWS
     if ragged:
         vec = vec_width(dt)
     u_ = "_u" if ragged else ""
