@@ -570,7 +570,14 @@ def row_split(nrows: int, N: int, vec: int, itemsize: int) -> RowSplit | None:
     return RowSplit(nch, segs, splits) if splits > 1 else None
 
 
-RAGGED_MIN_ROWS = 64
+def ragged_pays(nrows: int, N: int, itemsize: int) -> bool:
+    """Unaligned vectors for rows of no whole number of them?  Few rows are bound by one row's
+    latency, which one element per lane, on more lanes, shortens.  us, vectors / elements,
+    softmax: fp32 [37, 4097] 3.40 / 3.04, bf16 [300, 16385] 9.30 / 8.27, [600, 16385] 12.2 /
+    13.0, [600, 4097] 5.52 / 5.53, [3000, 4097] 12.3 / 17.7, fp32 [63, 32767] 7.02 / 7.85,
+    [200, 32767] 9.7 / 12.6, [300, 1001] 3.37 / 2.77, [3000, 1001] 5.02 / 6.33.  From 16 MB
+    memory sets the time whatever the rows."""
+    return nrows >= 512 or nrows >= 64 and N * itemsize >= 48 << 10 or nrows * N * itemsize >= 16 << 20
 
 
 def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[str, Launch]:
@@ -588,7 +595,7 @@ def gen_row(g: KernelGen, stages: list[Kernel], rows: tuple, N: int) -> tuple[st
     # twice to the same bits, counted once by a sum).  Against one element per lane (one box, us):
     # softmax bf16 [21409, 6269] 129.8 -> 89.5, LayerNorm 173.7 -> 92.9, RMSNorm fp32
     # [16384, 4095] 97.5 -> 74.7 (7.2 TB/s), LayerNorm bf16 [50000, 301] 51.0 -> 15.0.
-    ragged = vec == 1 and N >= vec_width(dt) and nrows >= RAGGED_MIN_ROWS
+    ragged = vec == 1 and N >= vec_width(dt) and ragged_pays(nrows, N, dt.itemsize)
     if ragged:
         vec = vec_width(dt)
     u_ = "_u" if ragged else ""

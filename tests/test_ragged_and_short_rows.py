@@ -42,7 +42,8 @@ def test_short_rows_share_a_wave_and_long_ragged_rows_compile():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", DTYPES)
-@pytest.mark.parametrize("rows,n", [(1, 9), (5, 17), (70, 1001), (3, 4097), (2, 12001), (2, 32767), (1, 300001), (33, 63)])
+@pytest.mark.parametrize("rows,n", [(1, 9), (5, 17), (70, 1001), (3, 4097), (2, 12001), (2, 32767), (1, 300001), (33, 63),
+                                    (511, 9), (512, 9), (513, 1001), (512, 4097), (64, 32767)])
 def test_ragged_rows_match_float64(dt, rows, n):
     """One element past and short of a vector, of a wave's chunks, of the 256 / 1024-lane
     layouts, and a split reduction: sums count the last chunk's shared elements once."""
@@ -55,6 +56,17 @@ def test_ragged_rows_match_float64(dt, rows, n):
     _close(tj.jit(lambda a: tj.mean(a * a, axis=-1))(x), (X * X).mean(-1), n)
     assert torch.equal(tj.jit(lambda a: tj.max(a, axis=-1))(x), x.amax(-1))
     _close(tj.jit(lambda a, b: a * b + tj.sigmoid(b))(x, g), X * G + torch.sigmoid(G), 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", DTYPES)
+def test_long_odd_row_split_over_workgroups(dt):
+    """One row past the size from which a few rows take unaligned vectors."""
+    n = (16 << 20) // torch.empty((), dtype=dt).element_size() + 3
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    x = (torch.randn(1, n, device=DEV, generator=gen) + 0.5).to(dt)
+    _close(tj.jit(lambda a: tj.mean(a, axis=-1))(x), x.double().mean(-1), n)
+    assert torch.equal(tj.jit(lambda a: tj.max(a, axis=-1))(x), x.amax(-1))
 
 
 @pytest.mark.gpu
