@@ -133,6 +133,12 @@ def ring_loop_lines(cfg, dt: DType, M: int, N: int, K: int, tb: bool, opvec: str
         out = ["{", f"  const unsigned int kt = {t0}({t});"]
         if guard_k:
             out.append(f"  const unsigned int kleft = kt * {BK}u < {K}u ? {K}u - kt * {BK}u : 0u;")
+            if KTs * S > KT:
+                # tiles past the end (a part with fewer K tiles): every lane's offset is OOB, and
+                # the scalar offset stays inside the descriptor, whose range check may subtract it
+                out[1] = out[1].replace("kt = ", "kf = ")
+                out[2] = out[2].replace("kt *", "kf *")
+                out.append(f"  const unsigned int kt = kf < {KT}u ? kf : {KT - 1}u;")
         for op, cnt in (("A", a_cnt), ("B", b_cnt)):
             row_k = op == "A" or tb
             step = BK * e if row_k else BK * N * e

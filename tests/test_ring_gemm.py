@@ -1,5 +1,7 @@
 """The ring-schedule GEMM: which products it takes, and its results at the edges of tiles, of
 K tiles and of K splits, on one stream and on several."""
+import re
+
 import pytest
 import torch
 
@@ -44,6 +46,29 @@ def test_ring_takes_whole_chunks_and_compiles(dt, tb):
         src, launches = hb.generate(p, {0: c})
         assert ("split_ws" in launches[0].meta) == (c.KSPLIT > 1)
         hb.compile_source(src, "gfx950")
+
+
+@pytest.mark.parametrize("tb", [True, False])
+@pytest.mark.parametrize("m,n,k,split", [(1, 64, 5 * 64, 3), (1, 64, 4 * 64 + 8, 3), (40, 72, 7 * 64, 4), (40, 72, 200, 1)])
+def test_k_tiles_past_the_end_keep_the_scalar_offset_in_range(m, n, k, tb, split):
+    """Parts with fewer K tiles load tiles past K: all lanes out of range (zeros), and the
+    scalar offset still below the operand's size, from which the range check may subtract it."""
+    src, _ = hb.generate(_program(m, n, k, tb, DType.bf16), {0: _ring(32, 64, 4, 2, 2, 4, split, DType.bf16)})
+    size = {op: int(r) for op, r in re.findall(r"rs([AB]) = __builtin_amdgcn_make_buffer_rsrc\(\(void\*\)[AB]b, \(short\)0, (\d+),", src)}
+    per = -(-(-(-k // 64)) // split)
+    blocks = re.findall(r"  \{\n((?:    const unsigned int k\w+ = [^\n]*\n)+)((?:    __builtin_amdgcn_raw_ptr_buffer_load_lds[^\n]*\n)+)", src)
+    assert len(blocks) >= per                                    # every tile of a part (none is in a loop here)
+    for head, loads in blocks:
+        for ksp in range(split):
+            env = {"kt0": ksp * per, "min": min}
+            for name, expr in re.findall(r"const unsigned int (\w+) = ([^\n]*);", head):
+                expr = re.sub(r"(\d+)u\b", r"\1", expr)
+                expr = re.sub(r"(.*?) < (.*?) \? (.*) : (.*)", r"(\3) if (\1) < (\2) else (\4)", expr)
+                env[name] = eval(expr, {}, env)
+            kf = env.get("kf", env["kt"])
+            assert env["kleft"] == max(0, k - kf * 64) if "kleft" in env else (kf + 1) * 64 <= k
+            for op, soff in re.findall(r"\(rs([AB]),.*, \(int\)\((.*?)\), 0, 0\);", loads):
+                assert eval(re.sub(r"(\d+)u\b", r"\1", soff), {}, env) < size[op], (op, ksp, kf)
 
 
 def test_ring_candidates_are_valid_and_bounded():
