@@ -1105,7 +1105,7 @@ def gen_colreduce(g: KernelGen) -> tuple[str, Launch | list[Launch]]:
 # many whole rows as fit (G of them, L vectors each), so its loads cover G * B consecutive
 # elements; the G partials of a column combine in a tree through LDS.  Split over S workgroups,
 # the last of them to finish folds the S partials (agent-coherent stores and loads, a counter in
-# the stream's workspace that is back at zero afterwards) and runs the finish: no second launch.
+# the stream's workspace that wraps to zero at the last count) and runs the finish: no second launch.
 # The plan's transpose and row reduction read and write the tensor twice more, and the transpose
 # of narrow rows gathers.  One box, us, plan -> here: bf16 [618418, 72] 1000 -> 24.3,
 # fp32 [177643, 30] 100 -> 10.4, [1000000, 16] 36.6 -> 17.2, bf16 [20000, 255] 31.2 -> 8.5,
@@ -1174,12 +1174,12 @@ def _colreduce_narrow(g: KernelGen, Rd: int, B: int, vec: int, L: int, S: int, R
               "  __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): this wave's partial stores are done",
               "  __shared__ unsigned int tj_last_;",
               "  __syncthreads();",
-              f"  if (tid == 0u) tj_last_ = atomicAdd(cnt_p, 1u) == {S - 1}u ? 1u : 0u;",
+              f"  if (tid == 0u) tj_last_ = atomicInc(cnt_p, {S - 1}u) == {S - 1}u ? 1u : 0u;   // {S - 1} wraps to 0",
               "  __syncthreads();", "  if (tj_last_ == 0u) return;",
               "#pragma unroll", f"  for (int q = 0; q < {vec}; ++q) acc[q] = {init};",
               f"  if (gi < {G}u) {{", "#pragma unroll 8", f"    for (unsigned int s2 = gi; s2 < {S}u; s2 += {G}u) {{",
               *ld, "    }", "  }",
-              *tree(), "  if (tid == 0u) *cnt_p = 0u;"]
+              *tree()]
     C += ["  if (gi != 0u) return;", "#pragma unroll", f"  for (int q = 0; q < {vec}; ++q) {{", "    const float a = acc[q];",
           f"    const {idx_t} r = {col_of} + q;"]
     C += finish_lines("r", "a", "    ") + ["  }", "}"]

@@ -252,8 +252,10 @@ def ring_split_lines(cfg, ntm: int, ntn: int, batch: int, bi: str) -> list[str]:
 
     The stores and loads are agent-coherent (sc1: past this XCD's L2), each wave waits for
     its stores before the workgroup barrier in front of the count, and the counters (at the
-    head of the stream's workspace block, zero when it is allocated) are back at zero after
-    every launch."""
+    head of the stream's workspace block, zero when it is allocated) wrap to zero at the last
+    count of a launch.  They are never stored to: whole launches that overlap in any order, which
+    only a caller that breaks run_static's rule can bring about, still leave them at zero, so
+    the damage ends with those launches."""
     S, nw = cfg.KSPLIT, cfg.num_warps
     TMW, TNW = cfg.TM // cfg.WM // 16, cfg.TN // cfg.WN // 16
     part = cfg.TM * cfg.TN * 4
@@ -269,7 +271,7 @@ def ring_split_lines(cfg, ntm: int, ntn: int, batch: int, bi: str) -> list[str]:
     L += ["  __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): this wave's partial stores are done",
           "  __shared__ unsigned int tj_last_;",
           "  __syncthreads();",
-          f"  if (tid == 0u) tj_last_ = atomicAdd(&cnt_p[ct_], 1u) == {S - 1}u ? 1u : 0u;",
+          f"  if (tid == 0u) tj_last_ = atomicInc(&cnt_p[ct_], {S - 1}u) == {S - 1}u ? 1u : 0u;   // {S - 1} wraps to 0",
           "  __syncthreads();",
           "  if (tj_last_ == 0u) return;"]
     for x in range(TMW):
@@ -281,7 +283,7 @@ def ring_split_lines(cfg, ntm: int, ntn: int, batch: int, bi: str) -> list[str]:
             L.append(f"    {{ const tj_f32x4 p = __builtin_bit_cast(tj_f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsW, "
                      f"(int)(wo_ + s * {part}u + {slot(x, y)}u), 0, 16));")
             L.append(f"      acc[{x}][{y}][0] += p[0]; acc[{x}][{y}][1] += p[1]; acc[{x}][{y}][2] += p[2]; acc[{x}][{y}][3] += p[3]; }}")
-    L += ["  }", "  if (tid == 0u) cnt_p[ct_] = 0u;"]
+    L.append("  }")
     return L
 
 

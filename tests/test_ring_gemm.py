@@ -94,6 +94,41 @@ def test_split_launches_share_the_workspace():
     assert args[1] == [(rt.WORKSPACE, 0, 32 * 4), (rt.WORKSPACE, 256, 4 * 32 * 32 * 32 * 4)]
 
 
+def _counter(src):
+    """(operation, limit, count of the last workgroup, whether the kernel stores to the counter)."""
+    (op, limit, last), = re.findall(r"tj_last_ = (atomic\w+)\(&?cnt_p(?:\[ct_\])?, (\d+)u\) == (\d+)u", src)
+    return op, int(limit), int(last), re.search(r"(\*cnt_p|cnt_p\[ct_\]) = ", src) is not None
+
+
+@pytest.mark.parametrize("kernel", ["ring", "columns"])
+def test_counters_return_to_zero_after_launches_that_overlap(kernel):
+    """Two launches on one counter, their workgroups' arrivals and (if the kernel has one) the
+    last one's later reset in every order: the counter ends at zero, so the next launch is right."""
+    if kernel == "ring":
+        src, _ = hb.generate(_program(64, 512, 1024, True, DType.bf16), {0: _ring(64, 64, 4, 2, 2, 4, 3, DType.bf16)})
+    else:
+        p = hb.fold_transpose_into_reduce(C.lower(tj.trace(lambda x: tj.sum(x, axis=0), [TensorType((700, 24), DType.f32)]), "hip"))
+        src, (launch,) = hb.generate(p)
+        assert launch.meta["splits"] > 1
+    op, limit, last, stores = _counter(src)
+    S = last + 1
+
+    def orders(value, left, resets):
+        if not any(left) and not resets:
+            yield value
+        for i in range(2):
+            if left[i]:
+                rest = [n - (j == i) for j, n in enumerate(left)]
+                after = value + 1 if op == "atomicAdd" else 0 if value >= limit else value + 1
+                yield from orders(after, rest, resets + (stores and value == last))
+        if resets:
+            yield from orders(0, left, resets - 1)
+
+    if S > 3:                                     # every order of two launches of three: the rule does not depend on S
+        limit, last, S = limit - S + 3, 2, 3
+    assert set(orders(0, [S, S], 0)) == {0}
+
+
 DEV = "cuda:0"
 
 
