@@ -42,7 +42,7 @@
 extern "C" {
 #endif
 
-#define TJ_HIP_ABI_VERSION 3
+#define TJ_HIP_ABI_VERSION 4
 
 /* Where a kernel argument points: caller input i, arena + offset, caller output j, or the
    program's workspace + offset.  The workspace holds what one launch keeps to itself (the

@@ -14,7 +14,7 @@ from typing import Sequence
 
 LIB_NAME = "libtjhip.so"
 LIB_PATH = Path(__file__).resolve().parents[1] / LIB_NAME
-ABI_VERSION = 3
+ABI_VERSION = 4
 
 INPUT, ARENA, OUTPUT, WORKSPACE = 0, 1, 2, 3
 STATIC_ARENA_BYTES = 64 << 20   # TJ_HIP_STATIC_ARENA_BYTES

@@ -33,6 +33,15 @@ def test_abi_version_matches():
     assert rt.load().tj_hip_abi_version() == rt.ABI_VERSION
 
 
+def test_argument_kinds_belong_to_the_abi_version():
+    """A library must not pass the version check and then refuse a program's argument kinds:
+    the kinds a version knows are fixed, and a further one takes a new version."""
+    kinds = dict(re.findall(r"TJ_ARG_(\w+) = (\d+)", HEADER.read_text()))
+    assert kinds == {"INPUT": "0", "ARENA": "1", "OUTPUT": "2", "WORKSPACE": "3"}
+    assert rt.ABI_VERSION == 4
+    assert (rt.INPUT, rt.ARENA, rt.OUTPUT, rt.WORKSPACE) == (0, 1, 2, 3)
+
+
 def test_compile_error_carries_the_hiprtc_log():
     with pytest.raises(rt.HipError) as e:
         rt.compile_source('extern "C" __global__ void k() { this is not hip; }', "bad.hip", ["--offload-arch=gfx950"])
