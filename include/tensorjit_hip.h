@@ -45,12 +45,13 @@ extern "C" {
 #define TJ_HIP_ABI_VERSION 4
 
 /* Where a kernel argument points: caller input i, arena + offset, caller output j, or the
-   program's workspace + offset.  The workspace holds what one launch keeps to itself (the
-   partials and tile counters of a product split over K): zero when allocated, one block per
-   stream that the program runs on (per stream and capture under stream capture, where the
-   block belongs to the captured graph's launches), one of its own for run_static, all freed
-   with the program.  The first is allocated with the program, a further stream's on its
-   first call. */
+   program's workspace + offset.  The workspace holds what one launch keeps to itself: its head,
+   everything below the lowest nonzero workspace offset, holds the tile counters of kernels
+   whose last workgroup sums (zero before a launch and after it), the rest their partials.
+   Launches get a workspace block of the stream they run on, under stream capture one of the
+   captured graph.  A stream keeps its block until the program is destroyed or more than 40
+   streams hold one; a graph's is the program's again once the graph, its execs and their
+   launches are gone (not by hipGraphExecUpdate: keep the graph an exec was updated from). */
 enum { TJ_ARG_INPUT = 0, TJ_ARG_ARENA = 1, TJ_ARG_OUTPUT = 2, TJ_ARG_WORKSPACE = 3 };
 
 typedef struct tj_argref {
@@ -75,6 +76,7 @@ typedef struct tj_stats {
   uint64_t graph_captures;
   uint64_t host_ns;          /* host time spent inside run/replay (launch overhead) */
   uint64_t direct_fallbacks; /* replay calls that launched directly (pointer sets not recurring) */
+  uint64_t workspace_blocks; /* workspace blocks held, free ones included */
 } tj_stats;
 
 typedef struct tj_device_info {
@@ -106,13 +108,17 @@ void tj_hip_free(void* p);
 /* Load the code object on `device`, resolve `nkernels` kernels, validate argument
  * references (args holds sum(launches[k].nargs) entries, kernel by kernel; every
  * ARENA reference must lie inside the arena: 0 < bytes and offset + bytes <=
- * arena_bytes) and allocate the arena with one hipMalloc. */
+ * arena_bytes) and allocate the arena with one hipMalloc, a program with a workspace also
+ * its first block and what tj_hip_program_run_static needs of one. */
 int tj_hip_program_create(int device, const void* code, size_t code_size, int nkernels,
                           const char* const* names, const tj_launch* launches, const tj_argref* args,
                           size_t arena_bytes, int n_inputs, int n_outputs, void** handle);
 
 /* Launch every kernel in order on `stream` (a hipStream_t; NULL = default stream).
- * Asynchronous: never synchronises. */
+ * Asynchronous: never waits for `stream`.  A program with a workspace allocates a block the
+ * first time it meets a second stream or capture: cleared in order on the stream, under
+ * capture on a stream of its own that the call waits for.  A 41st stream waits for the device
+ * once and reuses the other streams' blocks. */
 int tj_hip_program_run(void* handle, const void* const* inputs, void* const* outputs, void* stream);
 
 /* Allocation-free variant of tj_hip_program_run.  No counterpart in the reference: it
@@ -120,17 +126,23 @@ int tj_hip_program_run(void* handle, const void* const* inputs, void* const* out
  * serving loops, harnesses that forbid hipMalloc).  The program's intermediates and
  * split-K partials go to a static device array of TJ_HIP_STATIC_ARENA_BYTES per GPU
  * instead of the program's own arena; a program whose arena is larger is rejected
- * with an error.  The call allocates nothing: tj_hip_program_create looks the
+ * with an error (partials that no longer fit beside the intermediates have memory of their
+ * own, allocated with the program).  The call allocates nothing: tj_hip_program_create looks the
  * array's address up (once per device), so even a program's first call may be
  * issued under stream capture.  Every call on one GPU shares that array, which keeps
  * the last call's contents: calls that overlap on one GPU (two streams, two threads)
  * race.
- * Nothing in it needs clearing -- every call writes each intermediate before reading it. */
+ * Nothing in it needs clearing -- every call writes each intermediate before reading it.  The
+ * tile counters are the program's own and wrap to zero, so overlapping calls spoil their own
+ * outputs only, except in a program whose launches split K into different counts: there a
+ * counter may be left nonzero and spoil later run_static calls too. */
 #define TJ_HIP_STATIC_ARENA_BYTES ((size_t)64 << 20)
 int tj_hip_program_run_static(void* handle, const void* const* inputs, void* const* outputs, void* stream);
 
 /* Capture the launch sequence for this input/output pointer set into a hipGraph exec
- * (kept in a small per-program cache keyed by the pointer set). */
+ * (kept in a small per-program cache keyed by the pointer set).  In a program with a workspace
+ * the execs captured so share one block; the first stream that replays one owns it from then
+ * on, and another stream captures its own. */
 int tj_hip_program_capture(void* handle, const void* const* inputs, void* const* outputs);
 
 /* Replay the graph captured for this pointer set on `stream`, capturing it first if

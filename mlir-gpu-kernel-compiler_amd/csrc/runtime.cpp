@@ -4,7 +4,8 @@
 // kernel program.  At creation each kernel argument is resolved to
 //   INPUT  i   -> i-th caller input pointer
 //   ARENA  off -> arena base + off   (intermediate placed by the memory planner)
-//   WORKSPACE off -> this stream's workspace block + off (partials of products split over K)
+//   WORKSPACE off -> this stream's workspace block + off (counters and partials of kernels
+//                    whose last workgroup sums)
 //   OUTPUT j   -> j-th caller output pointer
 // and validated, so a call only fills small pointer tables and issues one
 // hipModuleLaunchKernel per kernel on the caller's stream.  The arena is a
@@ -66,6 +67,8 @@ int hip_fail(hipError_t e, const char* what) {
 
 constexpr int kMaxArgs = 64;
 constexpr size_t kMaxGraphs = 8;
+// stream blocks of one program before their streams are assumed gone (torch keeps 32 per device)
+constexpr size_t kMaxStreamBlocks = 40;
 constexpr int kMissLimit = 4;        // captures in a row before pointer sets must recur
 constexpr size_t kMaxSightings = 8;  // pointer sets seen once since then, most recent first
 
@@ -79,10 +82,45 @@ struct KernelRec {
   std::vector<void*> params;
 };
 
+// A workspace block and the stream, or the capture on a stream, whose launches use it.
+struct Block {
+  enum Use { kFree, kStream, kCapture, kExec };
+  char* base = nullptr;
+  Use use = kFree;             // kExec: of execs captured ahead, until one is replayed
+  hipStream_t stream = nullptr;
+  uint64_t thread = 0;         // of the per-thread default stream, one handle for a stream per thread
+  unsigned long long capture = 0;
+};
+
+// Blocks whose captured graph, its execs and their launches are gone.  Shared with the graphs'
+// user objects, which may outlive the program; their callbacks may not call into HIP.
+struct Returned {
+  std::mutex mu;
+  std::vector<char*> bases;
+};
+
+struct Lease {
+  std::shared_ptr<Returned> to;
+  char* base;
+};
+
+void end_lease(void* p) {
+  std::unique_ptr<Lease> lease(static_cast<Lease*>(p));
+  std::lock_guard<std::mutex> lock(lease->to->mu);
+  lease->to->bases.push_back(lease->base);
+}
+
+uint64_t thread_of(hipStream_t stream) {
+  static std::atomic<uint64_t> next{1};
+  static thread_local const uint64_t id = next.fetch_add(1);
+  return stream == hipStreamPerThread ? id : 0;
+}
+
 struct GraphRec {
   std::vector<const void*> key;  // inputs then outputs
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  Block* block = nullptr;        // the workspace block its launches use
 };
 
 // Restores the calling thread's current device on scope exit.
@@ -101,24 +139,35 @@ class DeviceScope {
   int prev_ = -1;
 };
 
+// Lets the calling thread allocate and clear memory while some stream is captured.
+class RelaxedCapture {
+ public:
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 struct Program {
   int device = 0;
   hipModule_t module = nullptr;
   std::vector<KernelRec> kernels;
   char* arena = nullptr;
   size_t arena_bytes = 0;
-  // workspace blocks (TJ_ARG_WORKSPACE): one per stream and capture the program runs on, so
-  // launches of one program on several streams do not share partials or tile counters
-  struct Block {
-    hipStream_t stream;
-    unsigned long long capture;  // capture id, 0 outside stream capture
-    bool claimed;
-    char* base;
-  };
-  size_t ws_bytes = 0;
-  std::vector<Block> blocks;
-  char* static_ws = nullptr;  // the block of tj_hip_program_run_static
+  // workspace (TJ_ARG_WORKSPACE): the head (tile counters) is zero between launches, the rest
+  // (partials) holds nothing.  A block per stream and per capture the program runs on, so
+  // launches of one program on several streams do not share partials or counters.  A stream is
+  // known by its handle: hipStreamDestroy waits for the stream's work (measured: 30 ms of it),
+  // so the next owner of a handle finds the block idle.
+  size_t ws_bytes = 0, ws_head = 0;
+  std::list<Block> blocks;
+  std::shared_ptr<Returned> returned = std::make_shared<Returned>();
   std::mutex ws_mu;
+  // tj_hip_program_run_static's counters and partials (these in the static arena behind the
+  // intermediates where they fit, else behind the counters)
+  char* static_head = nullptr;
+  char* static_body = nullptr;
   int n_in = 0, n_out = 0;
   hipStream_t capture_stream = nullptr;
   std::list<GraphRec> graphs;  // most recently used first
@@ -139,20 +188,20 @@ struct Program {
     if (capture_stream) (void)hipStreamDestroy(capture_stream);
     if (arena) (void)hipFree(arena);
     for (Block& b : blocks) (void)hipFree(b.base);
-    if (static_ws) (void)hipFree(static_ws);
+    if (static_head) (void)hipFree(static_head);
     if (module) (void)hipModuleUnload(module);
   }
 
-  // A zeroed workspace block.  Zeroed on a stream of its own, so that it also works while
-  // another stream is being captured (the caller relaxes the thread's capture mode).
-  int new_block(char** out) {
+  // `bytes` of device memory whose first ws_head are zero: cleared in order on `stream`, or,
+  // without one (at creation, under capture), on a stream of its own that is waited for.
+  int new_zeroed(size_t bytes, hipStream_t stream, bool ordered, char** out) {
     void* p = nullptr;
-    TJ_HIP(hipMalloc(&p, ws_bytes));
-    hipStream_t s = nullptr;
-    hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMemsetAsync(p, 0, ws_bytes, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (s) (void)hipStreamDestroy(s);
+    TJ_HIP(hipMalloc(&p, bytes));
+    hipStream_t own = nullptr;
+    hipError_t e = ordered ? hipSuccess : hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipMemsetAsync(p, 0, ws_head, ordered ? stream : own);
+    if (e == hipSuccess && !ordered) e = hipStreamSynchronize(own);
+    if (own) (void)hipStreamDestroy(own);
     if (e != hipSuccess) {
       (void)hipFree(p);
       return hip_fail(e, "workspace block");
@@ -161,54 +210,146 @@ struct Program {
     return 0;
   }
 
-  // The workspace block of `stream` (null when the program has no workspace).
-  int workspace_for(hipStream_t stream, char** out) {
-    *out = nullptr;
-    if (!ws_bytes) return 0;
+  // Make blocks free again whose captured graphs are gone.
+  void take_back() {
+    std::vector<char*> bases;
+    {
+      std::lock_guard<std::mutex> lock(returned->mu);
+      bases.swap(returned->bases);
+    }
+    for (char* base : bases)
+      for (Block& b : blocks)
+        if (b.base == base) b.use = Block::kFree;
+  }
+
+  // The block becomes free with the last of the graph, its execs and their launches.  Without
+  // a user object it stays the capture's until the program is destroyed.
+  void lend(hipStream_t stream, Block& b) {
+    hipStreamCaptureStatus status;
+    unsigned long long id;
+    hipGraph_t graph = nullptr;
+    const hipGraphNode_t* deps;
+    size_t ndeps;
+    hipUserObject_t object = nullptr;
+    if (hipStreamGetCaptureInfo_v2(stream, &status, &id, &graph, &deps, &ndeps) != hipSuccess || !graph) return;
+    Lease* lease = new Lease{returned, b.base};
+    if (hipUserObjectCreate(&object, lease, end_lease, 1, hipUserObjectNoDestructorSync) != hipSuccess) {
+      delete lease;
+      return;
+    }
+    if (hipGraphRetainUserObject(graph, object, 1, hipGraphUserObjectMove) != hipSuccess) {
+      lease->to = std::make_shared<Returned>();  // the release below must not free the block
+      (void)hipUserObjectRelease(object, 1);
+    }
+  }
+
+  // Every stream block free again, once the device has drained (destroyed streams' blocks
+  // among them); not while a capture forbids the wait.
+  void reclaim_streams() {
+    if (hipDeviceSynchronize() != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    for (Block& b : blocks)
+      if (b.use == Block::kStream) b.use = Block::kFree;
+  }
+
+  // What `stream` now asks of a block: its own, or its capture's.
+  static int wanted(hipStream_t stream, Block* out) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     unsigned long long id = 0;
     // the legacy stream cannot be captured, and asking it fails while another one is
     if (stream) TJ_HIP(hipStreamGetCaptureInfo(stream, &status, &id));
-    const unsigned long long capture = status == hipStreamCaptureStatusActive ? id : 0;
+    const bool capturing = status == hipStreamCaptureStatusActive;
+    *out = Block{nullptr, capturing ? Block::kCapture : Block::kStream, stream, thread_of(stream), capturing ? id : 0};
+    return 0;
+  }
+
+  // The workspace block of `stream` (null when the program has no workspace).
+  int workspace_for(hipStream_t stream, Block** out) {
+    *out = nullptr;
+    if (!ws_bytes) return 0;
+    Block want;
+    if (int rc = wanted(stream, &want)) return rc;
     std::lock_guard<std::mutex> lock(ws_mu);
+    take_back();
+    size_t streams = 0;
     for (Block& b : blocks) {
-      if (b.claimed && b.stream == stream && b.capture == capture) {
-        *out = b.base;
+      if (owns(b, want)) {
+        *out = &b;
+        return 0;
+      }
+      streams += b.use == Block::kStream;
+    }
+    const bool capturing = want.use == Block::kCapture;
+    RelaxedCapture relaxed;
+    if (!capturing && streams >= kMaxStreamBlocks) reclaim_streams();
+    const int rc = free_block(want, !capturing, out);
+    if (!rc && capturing) lend(stream, **out);
+    return rc;
+  }
+
+  // The block of execs captured ahead.
+  int exec_block(Block** out) {
+    *out = nullptr;
+    if (!ws_bytes) return 0;
+    Block want;
+    want.use = Block::kExec;
+    std::lock_guard<std::mutex> lock(ws_mu);
+    take_back();
+    for (Block& b : blocks) {
+      if (b.use == Block::kExec) {
+        *out = &b;
         return 0;
       }
     }
+    RelaxedCapture relaxed;
+    return free_block(want, false, out);
+  }
+
+  static bool owns(const Block& b, const Block& want) {
+    return b.use == want.use && b.stream == want.stream && b.thread == want.thread && b.capture == want.capture;
+  }
+
+  // A free block, or a new one, for `want`.
+  int free_block(const Block& want, bool ordered, Block** out) {
     for (Block& b : blocks) {
-      if (!b.claimed) {
-        b = Block{stream, capture, true, b.base};
-        *out = b.base;
+      if (b.use == Block::kFree) {
+        char* base = b.base;
+        b = want;
+        b.base = base;
+        *out = &b;
         return 0;
       }
     }
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-    char* base = nullptr;
-    const int rc = new_block(&base);
-    (void)hipThreadExchangeStreamCaptureMode(&mode);
-    if (rc) return rc;
-    blocks.push_back(Block{stream, capture, true, base});
-    *out = base;
+    Block made = want;
+    if (int rc = new_zeroed(ws_bytes, want.stream, ordered, &made.base)) return rc;
+    blocks.push_back(made);
+    *out = &blocks.back();
     return 0;
   }
 
   // Fill every kernel's pointer table; `base` is the arena the ARENA offsets refer to
-  // (the program's own, or the static one of tj_hip_program_run_static), `ws` the workspace.
-  void bind(const void* const* in, void* const* out, char* base, char* ws) {
+  // (the program's own, or the static one of tj_hip_program_run_static), `head` and `body`
+  // are the workspace's two parts.
+  void bind(const void* const* in, void* const* out, char* base, char* head, char* body) {
     for (KernelRec& k : kernels) {
       for (size_t i = 0; i < k.refs.size(); ++i) {
         const tj_argref& r = k.refs[i];
         switch (r.kind) {
           case TJ_ARG_INPUT: k.values[i] = const_cast<void*>(in[r.value]); break;
           case TJ_ARG_ARENA: k.values[i] = base + r.value; break;
-          case TJ_ARG_WORKSPACE: k.values[i] = ws + r.value; break;
+          case TJ_ARG_WORKSPACE:
+            k.values[i] = static_cast<size_t>(r.value) < ws_head ? head + r.value : body + (r.value - ws_head);
+            break;
           default: k.values[i] = out[r.value]; break;
         }
       }
     }
+  }
+
+  void bind(const void* const* in, void* const* out, const Block* b) {
+    bind(in, out, arena, b ? b->base : nullptr, b ? b->base + ws_head : nullptr);
   }
 
   int launch_one(KernelRec& k, hipStream_t stream) {
@@ -245,12 +386,23 @@ struct Program {
     return key;
   }
 
-  GraphRec* find(const std::vector<const void*>& key) {
+  // The exec of this pointer set that `want` may launch: without a workspace, or for an exec
+  // captured ahead (`want` null), any; else one whose launches use a block `want` owns.  An
+  // exec captured ahead gives its block to the first stream that replays it.
+  GraphRec* find(const std::vector<const void*>& key, const Block* want) {
     for (auto it = graphs.begin(); it != graphs.end(); ++it) {
-      if (it->key == key) {
-        graphs.splice(graphs.begin(), graphs, it);
-        return &graphs.front();
+      if (it->key != key) continue;
+      if (it->block && want) {
+        std::lock_guard<std::mutex> lock(ws_mu);
+        if (it->block->use == Block::kExec && want->use == Block::kStream) {
+          char* base = it->block->base;
+          *it->block = *want;
+          it->block->base = base;
+        }
+        if (!owns(*it->block, *want)) continue;
       }
+      graphs.splice(graphs.begin(), graphs, it);
+      return &graphs.front();
     }
     return nullptr;
   }
@@ -270,13 +422,16 @@ struct Program {
 
   // The exec for this pointer set, captured now if needed; *rec_out stays null when the
   // miss policy says to launch directly instead (only when `may_skip`).
-  // With a workspace the exec belongs to the stream it is launched on (its launches use that
-  // stream's block).
-  int capture(const void* const* in, void* const* out, hipStream_t stream, GraphRec** rec_out, bool may_skip = false) {
+  // With a workspace an exec belongs to the owner of the block its launches use: a stream's, or
+  // (`ahead`: no stream yet) that of the stream that first replays one captured ahead.
+  int capture(const void* const* in, void* const* out, hipStream_t stream, bool ahead, GraphRec** rec_out,
+              bool may_skip = false) {
     *rec_out = nullptr;
     std::vector<const void*> key = key_of(in, out);
-    if (ws_bytes) key.push_back(stream);
-    if (GraphRec* hit = find(key)) {
+    Block want;
+    if (ws_bytes && !ahead)
+      if (int rc = wanted(stream, &want)) return rc;
+    if (GraphRec* hit = find(key, ahead ? nullptr : &want)) {
       miss_streak = 0;
       *rec_out = hit;
       return 0;
@@ -286,11 +441,12 @@ struct Program {
       miss_streak++;
     }
     if (!capture_stream) TJ_HIP(hipStreamCreateWithFlags(&capture_stream, hipStreamNonBlocking));
-    char* ws = nullptr;
-    if (int rc = workspace_for(stream, &ws)) return rc;
-    bind(in, out, arena, ws);
+    Block* block = nullptr;
+    if (int rc = ahead ? exec_block(&block) : workspace_for(stream, &block)) return rc;
+    bind(in, out, block);
     GraphRec rec;
     rec.key = std::move(key);
+    rec.block = block;
     TJ_HIP(hipStreamBeginCapture(capture_stream, hipStreamCaptureModeThreadLocal));
     int rc = launch_all(capture_stream);
     hipError_t end = hipStreamEndCapture(capture_stream, &rec.graph);
@@ -468,6 +624,7 @@ int tj_hip_program_create(int device, const void* code, size_t code_size, int nk
         if (a.value < 0 || a.bytes <= 0 || a.bytes > (int64_t{1} << 40) || a.value > (int64_t{1} << 40))
           return fail("bad workspace buffer in " + rec.name);
         p->ws_bytes = std::max(p->ws_bytes, static_cast<size_t>(a.value + a.bytes));
+        if (a.value && (!p->ws_head || static_cast<size_t>(a.value) < p->ws_head)) p->ws_head = static_cast<size_t>(a.value);
       } else {
         return fail("bad argument kind in " + rec.name);
       }
@@ -492,21 +649,27 @@ int tj_hip_program_create(int device, const void* code, size_t code_size, int nk
     p->arena = static_cast<char*>(a);
   }
   if (p->ws_bytes) {
-    char* b = nullptr;
-    if (int rc = p->new_block(&b)) return rc;
-    p->blocks.push_back(Program::Block{nullptr, 0, false, b});
-    if (int rc = p->new_block(&p->static_ws)) return rc;
+    if (!p->ws_head) p->ws_head = p->ws_bytes;
+    Block b;
+    if (int rc = p->new_zeroed(p->ws_bytes, nullptr, false, &b.base)) return rc;
+    p->blocks.push_back(b);
   }
   // tj_hip_program_run_static's arena: looked up here, where loading and allocating are
   // expected, so that entry point never makes the runtime load or place anything.  A
   // failed lookup leaves the program usable through the other entry points.
-  if (arena_bytes && arena_bytes <= TJ_HIP_STATIC_ARENA_BYTES) {
+  if ((arena_bytes || p->ws_bytes) && arena_bytes <= TJ_HIP_STATIC_ARENA_BYTES) {
     const std::string saved = g_error;
     if (static_arena(device, &p->static_base) != 0) {
       p->static_error = g_error;
       p->static_base = nullptr;
       g_error = saved;
     }
+  }
+  if (p->ws_bytes && arena_bytes <= TJ_HIP_STATIC_ARENA_BYTES) {
+    const size_t at = (arena_bytes + 255) / 256 * 256;
+    const bool fits = p->static_base && at + (p->ws_bytes - p->ws_head) <= TJ_HIP_STATIC_ARENA_BYTES;
+    if (int rc = p->new_zeroed(fits ? p->ws_head : p->ws_bytes, nullptr, false, &p->static_head)) return rc;
+    p->static_body = fits ? p->static_base + at : p->static_head + p->ws_head;
   }
   *handle = p.release();
   return 0;
@@ -518,10 +681,10 @@ int tj_hip_program_run(void* handle, const void* const* inputs, void* const* out
   if ((p->n_in && !inputs) || (p->n_out && !outputs)) return fail("tj_hip_program_run: null pointer table");
   const uint64_t t0 = now_ns();
   DeviceScope scope(p->device);
-  char* ws = nullptr;
-  int rc = p->workspace_for(static_cast<hipStream_t>(stream), &ws);
+  Block* block = nullptr;
+  int rc = p->workspace_for(static_cast<hipStream_t>(stream), &block);
   if (rc) return rc;
-  p->bind(inputs, outputs, p->arena, ws);
+  p->bind(inputs, outputs, block);
   rc = p->launch_all(static_cast<hipStream_t>(stream));
   if (rc) return rc;
   p->stats.calls++;
@@ -542,7 +705,7 @@ int tj_hip_program_run_static(void* handle, const void* const* inputs, void* con
                 p->static_error);
   const uint64_t t0 = now_ns();
   DeviceScope scope(p->device);
-  p->bind(inputs, outputs, p->static_base, p->static_ws);
+  p->bind(inputs, outputs, p->static_base, p->static_head, p->static_body);
   int rc = p->launch_all(static_cast<hipStream_t>(stream));
   if (rc) return rc;
   p->stats.calls++;
@@ -556,7 +719,7 @@ int tj_hip_program_capture(void* handle, const void* const* inputs, void* const*
   if ((p->n_in && !inputs) || (p->n_out && !outputs)) return fail("tj_hip_program_capture: null pointer table");
   DeviceScope scope(p->device);
   GraphRec* rec = nullptr;
-  return p->capture(inputs, outputs, nullptr, &rec);
+  return p->capture(inputs, outputs, nullptr, /*ahead=*/true, &rec);
 }
 
 int tj_hip_program_replay(void* handle, const void* const* inputs, void* const* outputs, void* stream) {
@@ -566,16 +729,16 @@ int tj_hip_program_replay(void* handle, const void* const* inputs, void* const* 
   const uint64_t t0 = now_ns();
   DeviceScope scope(p->device);
   GraphRec* rec = nullptr;
-  int rc = p->capture(inputs, outputs, static_cast<hipStream_t>(stream), &rec, /*may_skip=*/true);
+  int rc = p->capture(inputs, outputs, static_cast<hipStream_t>(stream), /*ahead=*/false, &rec, /*may_skip=*/true);
   if (rc) return rc;
   if (rec) {
     TJ_HIP(hipGraphLaunch(rec->exec, static_cast<hipStream_t>(stream)));
     p->stats.graph_replays++;
   } else {
-    char* ws = nullptr;
-    rc = p->workspace_for(static_cast<hipStream_t>(stream), &ws);
+    Block* block = nullptr;
+    rc = p->workspace_for(static_cast<hipStream_t>(stream), &block);
     if (rc) return rc;
-    p->bind(inputs, outputs, p->arena, ws);
+    p->bind(inputs, outputs, block);
     rc = p->launch_all(static_cast<hipStream_t>(stream));
     if (rc) return rc;
     p->stats.direct_fallbacks++;
@@ -589,6 +752,9 @@ int tj_hip_program_stats(void* handle, tj_stats* out) {
   Program* p = as_program(handle);
   if (!p || !out) return fail("tj_hip_program_stats: null argument");
   *out = p->stats;
+  std::lock_guard<std::mutex> lock(p->ws_mu);
+  p->take_back();
+  out->workspace_blocks = p->blocks.size();
   return 0;
 }
 
@@ -609,9 +775,9 @@ int tj_hip_kernel_time(void* handle, int k, const void* const* inputs, void* con
   if ((p->n_in && !inputs) || (p->n_out && !outputs)) return fail("tj_hip_kernel_time: null pointer table");
   DeviceScope scope(p->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  char* ws = nullptr;
-  if (int wrc = p->workspace_for(s, &ws)) return wrc;
-  p->bind(inputs, outputs, p->arena, ws);
+  Block* block = nullptr;
+  if (int wrc = p->workspace_for(s, &block)) return wrc;
+  p->bind(inputs, outputs, block);
   KernelRec& kr = p->kernels[k];
   for (int i = 0; i < warmup; ++i)
     if (int rc = p->launch_one(kr, s)) return rc;
@@ -646,14 +812,14 @@ int tj_hip_program_time_kernels(void* handle, const void* const* inputs, void* c
   if (n == 0) return 0;
   DeviceScope scope(p->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  char* ws = nullptr;
-  if (int wrc = p->workspace_for(s, &ws)) return wrc;
+  Block* block = nullptr;
+  if (int wrc = p->workspace_for(s, &block)) return wrc;
   std::vector<hipEvent_t> ev(n + 1, nullptr);
   hipError_t e = hipSuccess;
   for (size_t i = 0; i <= n && e == hipSuccess; ++i) e = hipEventCreate(&ev[i]);
   int rc = 0;
   if (e == hipSuccess) {
-    p->bind(inputs, outputs, p->arena, ws);
+    p->bind(inputs, outputs, block);
     e = hipEventRecord(ev[0], s);
     for (size_t k = 0; k < n && e == hipSuccess && rc == 0; ++k) {
       rc = p->launch_one(p->kernels[k], s);

@@ -37,7 +37,7 @@ class LaunchDesc(ctypes.Structure):
 class Stats(ctypes.Structure):
     _fields_ = [("calls", ctypes.c_uint64), ("graph_replays", ctypes.c_uint64),
                 ("graph_captures", ctypes.c_uint64), ("host_ns", ctypes.c_uint64),
-                ("direct_fallbacks", ctypes.c_uint64)]
+                ("direct_fallbacks", ctypes.c_uint64), ("workspace_blocks", ctypes.c_uint64)]
 
 
 class DeviceInfo(ctypes.Structure):
@@ -233,7 +233,8 @@ class NativeHipProgram:
         s = Stats()
         check(self._lib.tj_hip_program_stats(self.handle, ctypes.byref(s)), "tj_hip_program_stats")
         return {"calls": s.calls, "graph_replays": s.graph_replays, "graph_captures": s.graph_captures,
-                "direct_fallbacks": s.direct_fallbacks, "host_us": s.host_ns / 1e3}
+                "direct_fallbacks": s.direct_fallbacks, "workspace_blocks": s.workspace_blocks,
+                "host_us": s.host_ns / 1e3}
 
     def arena(self) -> tuple[int, int]:
         p, n = ctypes.c_void_p(), ctypes.c_size_t()
