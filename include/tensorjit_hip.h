@@ -149,7 +149,8 @@ int tj_hip_program_capture(void* handle, const void* const* inputs, void* const*
  * this pointer set has not been seen.  After 4 captures in a row with no replay of a
  * cached exec (the caller keeps its outputs or passes fresh inputs), a pointer set is
  * captured on its second sighting only; calls in between launch the kernels directly
- * (counted in direct_fallbacks), so captures stay bounded. */
+ * (counted in direct_fallbacks), so captures stay bounded.  While `stream` is being captured
+ * every call launches the kernels directly, into the caller's graph (counted likewise). */
 int tj_hip_program_replay(void* handle, const void* const* inputs, void* const* outputs, void* stream);
 
 int tj_hip_program_stats(void* handle, tj_stats* out);

@@ -394,7 +394,7 @@ struct Program {
       if (it->key != key) continue;
       if (it->block && want) {
         std::lock_guard<std::mutex> lock(ws_mu);
-        if (it->block->use == Block::kExec && want->use == Block::kStream) {
+        if (it->block->use == Block::kExec) {
           char* base = it->block->base;
           *it->block = *want;
           it->block->base = base;
@@ -422,16 +422,12 @@ struct Program {
 
   // The exec for this pointer set, captured now if needed; *rec_out stays null when the
   // miss policy says to launch directly instead (only when `may_skip`).
-  // With a workspace an exec belongs to the owner of the block its launches use: a stream's, or
-  // (`ahead`: no stream yet) that of the stream that first replays one captured ahead.
-  int capture(const void* const* in, void* const* out, hipStream_t stream, bool ahead, GraphRec** rec_out,
-              bool may_skip = false) {
+  // With a workspace an exec belongs to the owner of the block its launches use: that of `want`,
+  // a stream outside capture, or (null) that of the stream that first replays one captured ahead.
+  int capture(const void* const* in, void* const* out, const Block* want, GraphRec** rec_out, bool may_skip = false) {
     *rec_out = nullptr;
     std::vector<const void*> key = key_of(in, out);
-    Block want;
-    if (ws_bytes && !ahead)
-      if (int rc = wanted(stream, &want)) return rc;
-    if (GraphRec* hit = find(key, ahead ? nullptr : &want)) {
+    if (GraphRec* hit = find(key, want)) {
       miss_streak = 0;
       *rec_out = hit;
       return 0;
@@ -442,7 +438,7 @@ struct Program {
     }
     if (!capture_stream) TJ_HIP(hipStreamCreateWithFlags(&capture_stream, hipStreamNonBlocking));
     Block* block = nullptr;
-    if (int rc = ahead ? exec_block(&block) : workspace_for(stream, &block)) return rc;
+    if (int rc = want ? workspace_for(want->stream, &block) : exec_block(&block)) return rc;
     bind(in, out, block);
     GraphRec rec;
     rec.key = std::move(key);
@@ -719,7 +715,7 @@ int tj_hip_program_capture(void* handle, const void* const* inputs, void* const*
   if ((p->n_in && !inputs) || (p->n_out && !outputs)) return fail("tj_hip_program_capture: null pointer table");
   DeviceScope scope(p->device);
   GraphRec* rec = nullptr;
-  return p->capture(inputs, outputs, nullptr, /*ahead=*/true, &rec);
+  return p->capture(inputs, outputs, nullptr, &rec);
 }
 
 int tj_hip_program_replay(void* handle, const void* const* inputs, void* const* outputs, void* stream) {
@@ -729,7 +725,10 @@ int tj_hip_program_replay(void* handle, const void* const* inputs, void* const* 
   const uint64_t t0 = now_ns();
   DeviceScope scope(p->device);
   GraphRec* rec = nullptr;
-  int rc = p->capture(inputs, outputs, static_cast<hipStream_t>(stream), /*ahead=*/false, &rec, /*may_skip=*/true);
+  Block want;
+  int rc = Program::wanted(static_cast<hipStream_t>(stream), &want);
+  // a graph launched on a stream under capture would run now and not be recorded
+  if (!rc && want.use != Block::kCapture) rc = p->capture(inputs, outputs, &want, &rec, /*may_skip=*/true);
   if (rc) return rc;
   if (rec) {
     TJ_HIP(hipGraphLaunch(rec->exec, static_cast<hipStream_t>(stream)));

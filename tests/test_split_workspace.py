@@ -131,6 +131,30 @@ def test_replayed_program_of_many_split_launches_on_several_streams():
     assert cp.stats["graph_replays"] >= 9 and cp.native_stats()["workspace_blocks"] <= 3
 
 
+@pytest.mark.parametrize("k", [192, 6144])               # without and with K splits
+def test_replayed_program_is_recorded_in_the_callers_capture(k):
+    """A program that replays graphs of its own, called under stream capture: its launches are
+    part of the captured graph, and eager calls on that stream stay right afterwards."""
+    fn = tj.jit(lambda w, *xs: tuple(tj.linear(x, w) for x in xs), tune=False)
+    gen = torch.Generator(device=DEV).manual_seed(0)
+    r = lambda *s: torch.randint(-2, 3, s, device=DEV, generator=gen).to(torch.bfloat16)  # noqa: E731
+    w, xs = r(256, k), [r(32, k) for _ in range(12)]
+    refs = [(x.double() @ w.double().t().contiguous()).to(torch.bfloat16) for x in xs]
+    assert fn.compiled(w, *xs).use_graph
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        outs = fn(w, *xs)
+    for _ in range(3):
+        for o in outs:
+            o.fill_(7)
+        graph.replay()
+        with torch.cuda.stream(side):
+            eager = fn(w, *xs)
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, t) and torch.equal(e, t) for o, e, t in zip(outs, eager, refs))
+
+
 def test_more_streams_than_blocks():
     prog, args, ref, _ = _split_program()
     outs = [torch.empty_like(ref) for _ in range(45)]
