@@ -28,7 +28,8 @@ from ..passes import Kernel, Program
 from ..passes.fusion import _finalize
 from ..passes.memory_planner import MemoryPlan, plan_memory
 from ..runtime import hip as rt
-from ..runtime.autotune import HIP_CANDIDATES, HIP_F32_CANDIDATES, MatmulConfig, autotune, cost_model, ring_candidates
+from ..runtime.autotune import (HIP_CANDIDATES, HIP_F32_CANDIDATES, MatmulConfig, autotune, beside_ring, cost_model,
+                                ring_candidates)
 from ..runtime.cache import AutotuneStore, CodeObjectCache
 from ..runtime.dtypes import TORCH_DTYPE
 from ..runtime.pool import BufferPool
@@ -51,8 +52,9 @@ COMPILE_OPTS = ("-O3", "-std=c++17", "-fno-strict-aliasing", *NO_PACKED_FP32)
 
 def _candidates(k: Kernel) -> list[MatmulConfig]:
     """Valid tilings of ``k``.  Where the ring schedule applies (both operands in whole
-    16-byte chunks) it replaces the register-staged schedules: over 164 random shapes one of
-    those was the fastest twice, both NN products of more than 0.2 TFLOP."""
+    16-byte chunks) it replaces the register-staged schedules, but for the 256x256 tiles of
+    products that no direct-to-LDS tile takes either (NN, and K no multiple of its K step;
+    at K up to 64, a single K tile, the ring is the faster)."""
     mm = k.anchor
     dt = compute_dtype(mm)
     M, N, K, tb = matmul_dims(mm)
@@ -61,7 +63,18 @@ def _candidates(k: Kernel) -> list[MatmulConfig]:
     ring = [c for c in ring_candidates(M, N, K, batch, dt.itemsize) if config_ok(c, dt, mm)]
     if not ring:
         return cands
-    return ring + [c for c in cands if c.DIRECT or c.SPLIT_K > 1]
+    staged = dt != DType.f32 and K > 64 and not any(c.DIRECT for c in cands)
+    return ring + [c for c in cands if c.DIRECT or c.SPLIT_K > 1 or staged and beside_ring(c)]
+
+
+def _rank(k: Kernel, cands: list[MatmulConfig]):
+    """The cost of a tiling of ``k`` among ``cands``."""
+    mm = k.anchor
+    M, N, K, tb = matmul_dims(mm)
+    batch = math.prod(mm.shape[:-2]) if len(mm.shape) > 2 else 1
+    kind = "hip_f32" if compute_dtype(mm) == DType.f32 else "hip"
+    ring_nt = tb if any(c.STAGES for c in cands) and any(beside_ring(c) for c in cands) else None
+    return lambda c: cost_model(c, M, N, K, kind, batch, ring_nt)
 
 
 def matmul_key(k: Kernel, arch: str) -> str:
@@ -73,12 +86,8 @@ def matmul_key(k: Kernel, arch: str) -> str:
 
 
 def analytic_config(k: Kernel) -> MatmulConfig:
-    mm = k.anchor
-    M, N, K, _ = matmul_dims(mm)
-    batch = math.prod(mm.shape[:-2]) if len(mm.shape) > 2 else 1
-    dt = compute_dtype(mm)
-    kind = "hip_f32" if dt == DType.f32 else "hip"
-    return min(_candidates(k), key=lambda c: cost_model(c, M, N, K, kind, batch))
+    cands = _candidates(k)
+    return min(cands, key=_rank(k, cands))
 
 
 # ---------------------------------------------------------------------------
@@ -571,8 +580,9 @@ class HipProgram:
             n = int(min(max(3, 2.0 / max(first, 1e-3)), 200))
             return run(warmup, n)
 
-        return autotune(key, _candidates(k), build, (M, N, K, batch), kind, store=store, timer=timer, top_k=6,
-                        rounds=3)
+        cands = _candidates(k)
+        return autotune(key, cands, build, (M, N, K, batch), kind, store=store, timer=timer, top_k=6, rounds=3,
+                        rank=_rank(k, cands))
 
     # -- protocol ---------------------------------------------------------------
     @property

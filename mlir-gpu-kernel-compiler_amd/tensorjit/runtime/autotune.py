@@ -257,6 +257,42 @@ def _direct_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: in
     return 1.5 + max(t, _hbm_us(M, N, K, batch, elem) / 7.0)
 
 
+# The register-staged tilings that still beat the ring where no direct-to-LDS tile applies:
+# 256x256 with 8 waves, K step 32 or 64.  (NT, PINGPONG) -> us per K step of a round, us per
+# round beside its K loop, and the loss (M, N) from a last tile that is cut.  us, 16-bit, ring
+# (128x128) / the best of these:
+#   NN 8192^3 1005 / 921, 16384 x 4096 x 4096 519 / 485, 1000 x 16384 x 4096 136 / 125, 64 of
+#   512^3 38.5 / 25.9; but 2048 x 4096 x 4096 66 / 77, 2048 x 11008 x 4096 188 / 209, 6000^3
+#   462 / 531 (half-empty rounds of workgroups)
+#   NT with K no multiple of 64: 8192 x 8192 x 8200 1254 / 916, 2048 x 11008 x 4104 242 / 192,
+#   900 x 11008 x 4104 121 / 107; but 1500 x 11008 x 2056 108 / 116
+# No smaller staged tile, and none in fp32, was the fastest of 63 shapes.  Of 60 further random
+# shapes at which the two estimates are close, the choice is the slower one at 7, always the
+# ring: by 7-15%, and at 84 x 1152 x 184 x 496 62 / 43.
+STAGED_US = {
+    (False, 1): (0.915, 6.6, 1.0, 1.0), (False, 2): (0.910, 6.6, 1.17, 1.17), (False, 3): (2.3, 9.0, 1.5, 1.5),
+    (True, 1): (0.96, 4.0, 1.0, 1.0), (True, 2): (0.968, 8.0, 1.12, 1.12), (True, 3): (1.66, 10.0, 1.08, 1.3),
+}
+
+
+def beside_ring(cfg: MatmulConfig) -> bool:
+    """A register-staged tiling that is kept where the ring schedule applies too."""
+    return cfg.PINGPONG > 0 and (cfg.TM, cfg.TN, cfg.WM, cfg.TK) == (256, 256, 2, 64 if cfg.PINGPONG == 3 else 32)
+
+
+def _staged_us(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, tb: bool) -> float:
+    """Microseconds of a ``beside_ring`` tiling: whole rounds of one workgroup per CU; a last
+    round that is not full runs at a higher clock and rate."""
+    step, epi, cut_m, cut_n = STAGED_US[(tb, cfg.PINGPONG)]
+    wgs = -(-M // cfg.TM) * -(-N // cfg.TN) * batch
+    rounds = -(-wgs // CU_COUNT)
+    last = 0.7 + 0.3 * (wgs - (rounds - 1) * CU_COUNT) / CU_COUNT
+    cut = max(cut_m if M % cfg.TM else 1.0, cut_n if N % cfg.TN else 1.0)
+    # what the estimate misses: a launch's start, few K steps, output rows off the 128-byte lines
+    lead = (1.24 if not tb and N % 64 else 1.0) / (0.93 if K < 256 else 1.0)
+    return ((rounds - 1 + last) * (-(-K // cfg.TK) * step + epi) * cut + 2.0) * lead
+
+
 def _skinny_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
     """Streaming kernel (M <= 16 / 32), from 35 shapes of 1-16 rows on MI355X: HBM, or rounds
     of one workgroup per CU whose waves each run K / SPLIT_K serially (8 waves of 16 columns
@@ -344,9 +380,18 @@ def _hip_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) 
     return t * 1e6
 
 
-def cost_model(cfg: MatmulConfig, M: int, N: int, K: int, backend: str, batch: int = 1) -> float:
+def cost_model(cfg: MatmulConfig, M: int, N: int, K: int, backend: str, batch: int = 1,
+               ring_nt: bool | None = None) -> float:
     """Lower is better.  ``backend``: "hip" (bf16/fp16) or "hip_f32"; CPU kinds
-    "c" / "c_dot" keep the reference's register-pressure heuristic."""
+    "c" / "c_dot" keep the reference's register-pressure heuristic.  ``ring_nt``: whether B is
+    stored [N][K], given where ring and register-staged tilings compete."""
+    if backend == "hip" and ring_nt is not None:
+        if cfg.PINGPONG:
+            return _staged_us(cfg, M, N, K, batch, ring_nt)
+        if cfg.STAGES:
+            # the ring beside these: 0.91 of its model, or where B's rows start inside a
+            # 128-byte line 1.13 (NT) and 1.06 (NN)
+            return _hip_cost(cfg, M, N, K, batch, 2) * (1.13 if ring_nt else 1.06 if N % 64 else 0.91)
     if backend in ("hip", "hip_f32"):
         return _hip_cost(cfg, M, N, K, batch, 2 if backend == "hip" else 4)
     tm, tn = cfg.TM, cfg.TN
@@ -387,6 +432,7 @@ def autotune(
     iters: int = 5,
     timer: Callable[[Callable[[], None], int, int], float] | None = None,
     rounds: int = 1,
+    rank: Callable[[MatmulConfig], float] | None = None,
 ) -> MatmulConfig:
     """Fastest candidate by measurement; ``build(cfg)`` returns a runner for ``timer``.
 
@@ -394,12 +440,12 @@ def autotune(
     GPU kernels).  All runners are built first, then timed in ``rounds`` interleaved
     passes keeping each candidate's best time, so clock ramp-up or a noisy
     neighbour cannot favour whichever candidate happened to run last.  Candidates
-    whose build or run raises are skipped.
+    whose build or run raises are skipped.  ``rank`` replaces the cost model's order.
     """
     store = store or AutotuneStore()
     M, N, K = shape[:3]
     batch = shape[3] if len(shape) > 3 else 1
-    rank = lambda c: cost_model(c, M, N, K, backend, batch)  # noqa: E731
+    rank = rank or (lambda c: cost_model(c, M, N, K, backend, batch))
     if os.environ.get("TENSORJIT_NO_AUTOTUNE") == "1":
         return min(candidates, key=rank)
     cached = store.get(key)

@@ -81,6 +81,32 @@ def test_ring_candidates_are_valid_and_bounded():
                 assert launch.meta["lds_bytes"] <= 160 * 1024 and launch.grid[2] == c.KSPLIT
 
 
+@pytest.mark.parametrize("m,n,k,tb,lead,staged", [
+    (8192, 8192, 8192, False, (), True), (4096, 4096, 16384, False, (), True), (16384, 4096, 4096, False, (), True),
+    (512, 512, 512, False, (64,), True), (8192, 8192, 8200, True, (), True), (2048, 11008, 4104, True, (), True),
+    (2048, 4096, 4096, False, (), False), (2048, 11008, 4096, False, (), False), (1000, 4096, 4104, True, (), False)])
+def test_products_without_a_direct_tile_keep_the_256_wide_staged_ones(m, n, k, tb, lead, staged):
+    """The choice without tuning, and what tuning may time: products of whole rounds of 256x256
+    tiles, where the ring's 128x128 measured 4-30% slower, and ones where it is the faster."""
+    dt = DType.bf16
+    b = TensorType((*lead, k, n) if not tb else (n, k), dt)
+    types = [TensorType((*lead, m, k), dt), b, TensorType((n,), dt)]
+    (kernel,) = C.lower(tj.trace(_fn(tb), types), "hip").kernels
+    cands = hb._candidates(kernel)
+    assert any(c.PINGPONG and (c.TM, c.TN) == (256, 256) for c in cands) and any(c.STAGES for c in cands)
+    cfg = hb.analytic_config(kernel)
+    assert (cfg.PINGPONG > 0) == staged and (cfg.STAGES > 0) == (not staged), cfg
+    top = sorted(cands, key=hb._rank(kernel, cands))[:6]
+    assert any(c.STAGES for c in top) and (not staged or sum(c.PINGPONG > 0 for c in top) >= 2)
+
+
+def test_products_with_a_direct_tile_time_no_staged_ones():
+    (kernel,) = _program(2048, 4096, 4096, True, DType.bf16).kernels
+    assert all(c.STAGES or c.DIRECT or c.SPLIT_K > 1 for c in hb._candidates(kernel))
+    (kernel,) = _program(4096, 4096, 4096, False, DType.f32).kernels
+    assert all(c.STAGES for c in hb._candidates(kernel))
+
+
 def test_split_launches_share_the_workspace():
     """Counters at the head of the block, as many as any launch has; partials behind them."""
     dt = DType.bf16
