@@ -74,7 +74,8 @@ def _rank(k: Kernel, cands: list[MatmulConfig]):
     batch = math.prod(mm.shape[:-2]) if len(mm.shape) > 2 else 1
     kind = "hip_f32" if compute_dtype(mm) == DType.f32 else "hip"
     ring_nt = tb if any(c.STAGES for c in cands) and any(beside_ring(c) for c in cands) else None
-    return lambda c: cost_model(c, M, N, K, kind, batch, ring_nt)
+    mats = tuple(math.prod(n.shape[:-2]) for n in mm.inputs)
+    return lambda c: cost_model(c, M, N, K, kind, batch, ring_nt, mats)
 
 
 def matmul_key(k: Kernel, arch: str) -> str:

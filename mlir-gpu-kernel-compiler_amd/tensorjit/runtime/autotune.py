@@ -188,11 +188,14 @@ RING_TILES = [
 ]
 
 
-def _hbm_us(M: int, N: int, K: int, batch: int, elem: int) -> float:
-    return (M * K + N * K + M * N) * batch * elem * 1e-6
+def _hbm_us(M: int, N: int, K: int, batch: int, elem: int, mats: tuple[int, int] | None = None) -> float:
+    """``mats``: distinct A and B matrices of the batch (a weight shared by all is read once)."""
+    na, nb = mats or (batch, batch)
+    return (M * K * na + N * K * nb + M * N * batch) * elem * 1e-6
 
 
-def _ring_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
+def _ring_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
+               mats: tuple[int, int] | None = None) -> float:
     """Microseconds of a ring-schedule product, fitted to 4.5k measured (shape, tiling) pairs
     over 205 random decode, prompt and MLP shapes in bf16, fp16 and fp32, NT and NN (rms error
     10% over the near-best tilings).  The busiest CU runs ``w`` workgroups, ``occ`` at a time;
@@ -209,7 +212,7 @@ def _ring_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int)
     t_dma = w * per * (tm + tn) * 0.128 * 0.0085
     t_lat = rounds * per * 0.1 / (cfg.STAGES - 1) ** 0.89
     # weights of up to ~64 MB come from the MALL on a repeated call; more stream from HBM
-    mem = _hbm_us(M, N, K, batch, elem)
+    mem = _hbm_us(M, N, K, batch, elem, mats)
     t_hbm = mem / 9.42
     edge = 4.0 if N % (16 // elem) else 1.0                       # element-wise stores of ragged rows
     t_epi = rounds * (0.62 + tm * tn * 1e-3 * 0.104 * conc * edge)
@@ -230,7 +233,8 @@ DIRECT_US = {
 PERSIST_US = {(256, 256): (0.879, 25.3), (256, 128): (0.737, 9.3)}
 
 
-def _direct_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
+def _direct_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
+                 mats: tuple[int, int] | None = None) -> float:
     """Microseconds of a direct-to-LDS product: whole rounds of ``occ`` workgroups per CU, then
     the last round at the concurrency it has left."""
     tm, tn = cfg.TM, cfg.TN
@@ -254,7 +258,7 @@ def _direct_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: in
     last = -(-(wgs - (rounds - 1) * CU_COUNT * occ) // CU_COUNT)
     step = one + (full - one) * (last - 1) / (occ - 1) if occ > 1 else full
     t = (rounds - 1) * (per * full + epi) + per * step + epi * last / occ
-    return 1.5 + max(t, _hbm_us(M, N, K, batch, elem) / 7.0)
+    return 1.5 + max(t, _hbm_us(M, N, K, batch, elem, mats) / 7.0)
 
 
 # The register-staged tilings that still beat the ring where no direct-to-LDS tile applies:
@@ -293,7 +297,8 @@ def _staged_us(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, tb: bool) 
     return ((rounds - 1 + last) * (-(-K // cfg.TK) * step + epi) * cut + 2.0) * lead
 
 
-def _skinny_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
+def _skinny_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
+                 mats: tuple[int, int] | None = None) -> float:
     """Streaming kernel (M <= 16 / 32), from 35 shapes of 1-16 rows on MI355X: HBM, or rounds
     of one workgroup per CU whose waves each run K / SPLIT_K serially (8 waves of 16 columns
     0.83 ns per k, 4 or 2 waves of 32 columns 1.9)."""
@@ -305,8 +310,12 @@ def _skinny_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: in
         per_k *= 1.3                                              # A is read in fragments, not through LDS
     if cfg.TM == 32:
         per_k *= 2.2
+    if mats and mats[1] < batch:
+        # a batch that shares its weight: [64, 1, 4096] x 4096 242 us where the ring takes 88,
+        # [2, 1, 4096] x 4096 9.6 (8.2), [16, 16, 1024] x 1024 5.8 (4.0)
+        per_k *= 1.7
     extra = {4: 1.0, 2: 1.04, 8: 1.06, 16: 1.1}.get(cfg.SPLIT_K, 1.2) * (1.0 if cfg.TN <= 32 else 1.05)
-    return 1.5 + max(rounds * K * per_k, _hbm_us(M, N, K, batch, elem) / 6.85) * extra
+    return 1.5 + max(rounds * K * per_k, _hbm_us(M, N, K, batch, elem, mats) / 6.85) * extra
 
 
 def _sched_factor(cfg: MatmulConfig) -> float:
@@ -324,13 +333,14 @@ def _sched_factor(cfg: MatmulConfig) -> float:
     return {3: 1.0, 2: 1.04, 1: 1.05}.get(cfg.PINGPONG, 1.09)
 
 
-def _hip_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) -> float:
+def _hip_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
+              mats: tuple[int, int] | None = None) -> float:
     if cfg.SPLIT_K > 1:
-        return _skinny_cost(cfg, M, N, K, batch, elem)
+        return _skinny_cost(cfg, M, N, K, batch, elem, mats)
     if cfg.STAGES:
-        return _ring_cost(cfg, M, N, K, batch, elem)
+        return _ring_cost(cfg, M, N, K, batch, elem, mats)
     if cfg.DIRECT:
-        return _direct_cost(cfg, M, N, K, batch, elem)
+        return _direct_cost(cfg, M, N, K, batch, elem, mats)
     tm, tn, tk = cfg.TM, cfg.TN, cfg.TK or 32
     waves = cfg.num_warps
     if cfg.SPLIT_K == 1 and (tm % (cfg.WM * cfg.MI) or tn % (cfg.WN * cfg.MI)):
@@ -381,19 +391,20 @@ def _hip_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int) 
 
 
 def cost_model(cfg: MatmulConfig, M: int, N: int, K: int, backend: str, batch: int = 1,
-               ring_nt: bool | None = None) -> float:
+               ring_nt: bool | None = None, mats: tuple[int, int] | None = None) -> float:
     """Lower is better.  ``backend``: "hip" (bf16/fp16) or "hip_f32"; CPU kinds
     "c" / "c_dot" keep the reference's register-pressure heuristic.  ``ring_nt``: whether B is
-    stored [N][K], given where ring and register-staged tilings compete."""
+    stored [N][K], given where ring and register-staged tilings compete; ``mats``: distinct A
+    and B matrices of the batch (default: as many as products)."""
     if backend == "hip" and ring_nt is not None:
         if cfg.PINGPONG:
             return _staged_us(cfg, M, N, K, batch, ring_nt)
         if cfg.STAGES:
             # the ring beside these: 0.91 of its model, or where B's rows start inside a
             # 128-byte line 1.13 (NT) and 1.06 (NN)
-            return _hip_cost(cfg, M, N, K, batch, 2) * (1.13 if ring_nt else 1.06 if N % 64 else 0.91)
+            return _hip_cost(cfg, M, N, K, batch, 2, mats) * (1.13 if ring_nt else 1.06 if N % 64 else 0.91)
     if backend in ("hip", "hip_f32"):
-        return _hip_cost(cfg, M, N, K, batch, 2 if backend == "hip" else 4)
+        return _hip_cost(cfg, M, N, K, batch, 2 if backend == "hip" else 4, mats)
     tm, tn = cfg.TM, cfg.TN
     tk = cfg.TK or K
     cost = (4.0 * (tm * tk + tk * tn)) / (2.0 * tm * tn * tk)

@@ -100,6 +100,22 @@ def test_products_without_a_direct_tile_keep_the_256_wide_staged_ones(m, n, k, t
     assert any(c.STAGES for c in top) and (not staged or sum(c.PINGPONG > 0 for c in top) >= 2)
 
 
+SHARED = [((64, 1), 4096, 4096), ((16, 4), 4096, 4096), ((32, 1), 11008, 4096), ((8, 16), 4096, 4096),
+          ((128, 1), 1024, 1024), ((2, 1), 4096, 4096), ((32, 17), 1024, 4096)]
+
+
+@pytest.mark.parametrize("lead,n,k", SHARED)
+@pytest.mark.parametrize("dt", [DType.bf16, DType.f16])
+def test_batches_with_a_shared_weight_take_tiles_of_their_few_rows(lead, n, k, dt):
+    """A batch of a few rows each with one weight: the weight counts once, so that the tile
+    decides and not a floor that every tiling shares (which chose 192x256 for one row)."""
+    (kernel,) = _program(lead[-1], n, k, True, dt, lead[:-1]).kernels
+    cfg = hb.analytic_config(kernel)
+    assert cfg.STAGES and cfg.TM == 32, cfg
+    costs = sorted(hb._rank(kernel, hb._candidates(kernel))(c) for c in hb._candidates(kernel))
+    assert costs[0] < costs[1] or costs[1] < costs[-1] / 2       # the estimates differ
+
+
 def test_products_with_a_direct_tile_time_no_staged_ones():
     (kernel,) = _program(2048, 4096, 4096, True, DType.bf16).kernels
     assert all(c.STAGES or c.DIRECT or c.SPLIT_K > 1 for c in hb._candidates(kernel))
@@ -219,6 +235,16 @@ def test_ring_gemm_batched_and_epilogue_operand():
     prog = _native(lambda x, w: x + tj.linear(x, w), [x, w], _ring(32, 32, 4, 2, 2, 4, 1, dt))
     prog.run([x.data_ptr(), w.data_ptr()], [out.data_ptr()], torch.cuda.current_stream().cuda_stream)
     assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lead,n,k", [((64, 1), 512, 1024), ((16, 4), 264, 1000), ((8, 16), 512, 768), ((3, 300), 392, 192),
+                                      ((2, 3, 1), 768, 768)])
+@pytest.mark.parametrize("dt", [DType.bf16, DType.f16, DType.f32])
+def test_batches_with_a_shared_weight_through_the_chosen_tile(lead, n, k, dt):
+    args, ref = _integers(lead[-1], n, k, True, dt, lead=lead[:-1])
+    fn = tj.jit(_fn(True), tune=False)
+    assert torch.equal(fn(*args), ref) and torch.equal(fn(*args), ref), fn.compiled(*args).matmul_configs
 
 
 @pytest.mark.gpu
