@@ -358,24 +358,32 @@ def _split_counts(KB: int) -> list[int]:
     return [n for n in range(2, 33) if KB // n >= (2 if KB % n == 0 else 3)]
 
 
-def key_splits(tiles: int, KB: int, pingpong: bool, dims: int, out_elems: int) -> int:
+def key_splits(tiles: int, KB: int, pingpong: bool, dims: int, out_elems: int, alone: bool = True) -> int:
     """The split count of the least estimated time, for ``dims`` = D + Dv and ``out_elems``
     outputs.  A CU's second workgroup takes as long as its first (2.85 against 1.27 us per key
     block at head dim 128), so splits pay only by reaching idle CUs, and the fp32 partials
     cost 2.7 us and 0.58 us per MB.  us in 1 / 2 / 3 / 4 parts (the estimate's choice first):
     8 heads x 1100 x 128 3: 20.8 (25.7 / 22.1 / - / 27.3), 8 x 1850 x 64 2: 19.2 (21.7 / - /
     22.4 / 21.8), 64 x 330 x 64 1: 7.9 (- / 15.3 / 18.9), 32 x 600 x 128 1: 19.4 (- / 26.9 /
-    23.8 / 28.8), 8 x 2600 x 128 1: 52.9 (- / 55.5 / 47.8 / 54.5)."""
+    23.8 / 28.8), 8 x 2600 x 128 1: 52.9 (- / 55.5 / 47.8 / 54.5).  ``alone``: see ``_host_us``."""
     most = attention_splits(tiles, KB, pingpong)
     if most == 1 or os.environ.get("TENSORJIT_HIP_ATTENTION_SPLITS", "").isdigit():
         return most
 
-    def cost(n: int) -> float:
+    def cost(n: int) -> tuple[float, float]:
         kernel_us = 2.3 + -(-tiles * n // CU_COUNT) * -(-KB // n) * (0.23 + 1.04 * dims / 256)
-        # a call of one launch takes the host 7.7 us, of two 10.2
-        return max(7.7, kernel_us) if n == 1 else max(10.2, kernel_us + 2.7 + 0.58e-6 * out_elems * 4 * n)
+        kernel_us += 2.7 + 0.58e-6 * out_elems * 4 * n if n > 1 else 0.0
+        return max(kernel_us, _host_us(n, alone)), kernel_us
 
     return min([1] + [n for n in _split_counts(KB) if n <= most], key=cost)
+
+
+def _host_us(n: int, alone: bool) -> float:
+    """The host's time for a call of an attention kernel in ``n`` parts, which the call takes at
+    least where the kernel is a program of its own, launched eagerly.  Among the other kernels
+    of a program it is hidden, or part of a replayed graph (us in 1 / 6 parts, eager and in a
+    captured graph: 32 heads x 1 query x 1500 keys x 64 8.4 / 10.7, 8.4 / 5.3)."""
+    return 0.0 if not alone else 7.7 if n == 1 else 10.2
 
 
 def few_queries(Sq: int) -> bool:
@@ -389,35 +397,34 @@ def few_queries(Sq: int) -> bool:
 FEW_BLOCK = 32      # keys a wave takes at a time: one k step of the 16x16x32 PV MFMA
 
 
-def few_query_splits(batch: int, Sk: int, D: int, Dv: int) -> int:
+def few_query_splits(batch: int, Sk: int, D: int, Dv: int, alone: bool = True) -> int:
     """Key-range splits of the few-query kernel: the count of the least estimated time.  The
     kernel takes its bytes at a rate that grows with the workgroups resident (two per CU, four
     at head dims up to 64: their LDS tiles), or its steps of 128 keys one after the other;
     splits add a combine launch.  Measured: 320 heads x 3000 keys x 128 89.5 us in one part, 77.7
     in two, 75.4 in three (the fuller grid evens out the CUs); 512 heads x 4000 keys 152.8 in
-    one, 155.3 in two; 8 heads x 8192 keys 53.2 in one, 10.5 in 16.  Calls below
-    8 us are bound by the host's launch instead, which a second launch lengthens: 32 heads x
-    1500 keys x 64 8.5 us in one part, 10.5 in two."""
+    one, 155.3 in two; 8 heads x 8192 keys 53.2 in one, 10.5 in 16.  ``alone``: see
+    ``_host_us``; at equal calls the count of the shorter kernel."""
     forced = os.environ.get("TENSORJIT_HIP_ATTENTION_SPLITS", "")
     blocks = -(-Sk // FEW_BLOCK)
     if forced.isdigit():
-        return max(1, min(int(forced), blocks))
+        return max(1, min(int(forced), 32, blocks))
     slots = CU_COUNT * (2 if D + Dv > 128 else 4)
     step_us = 0.55 + 0.27 * (D + Dv) / 256
 
-    def cost(n: int) -> float:
+    def cost(n: int) -> tuple[float, float]:
         steps, groups = -(-(-(-blocks // n)) // 4), batch * n
         resident = min(groups, slots)
         rate = 7e6 * resident / (resident + 75)     # bytes per us: 5.7 TB/s at 320 workgroups
         stream_us = groups * steps * 4 * FEW_BLOCK * (D + Dv) * 2 / rate
         kernel_us = max(stream_us, -(-groups // slots) * steps * step_us) + (2.5 + 0.02 * n if n > 1 else 0.0)
-        return max(kernel_us, 7.7 if n == 1 else 10.2)
+        return max(kernel_us, _host_us(n, alone)), kernel_us
 
     return min((n for n in range(1, 33) if n == 1 or blocks >= 4 * n), key=cost)
 
 
 def _gen_few_queries(fname: str, dt: DType, batch: int, Sq: int, Sk: int, D: int, Dv: int, scale: float,
-                     q: tuple[str, int], k: tuple[str, int], v: tuple[str, int], o: tuple[str, int]):
+                     q: tuple[str, int], k: tuple[str, int], v: tuple[str, int], o: tuple[str, int], alone: bool):
     """Attention of at most 16 queries per head: bound by reading K and V once.
 
     A workgroup of 4 waves owns one (batch, head), or one split of its keys.  Blocks of 32
@@ -440,7 +447,7 @@ def _gen_few_queries(fname: str, dt: DType, batch: int, Sq: int, Sk: int, D: int
     (qoff, qst), (koff, kst), (voff, vst), (ooff, ost) = q, k, v, o
     T = CTYPE[dt]
     KB = -(-Sk // FEW_BLOCK)
-    NS = few_query_splits(batch, Sk, D, Dv)
+    NS = few_query_splits(batch, Sk, D, Dv, alone)
     KBL = -(-KB // NS)
     NS = -(-KB // KBL)                          # every split has a block
     idx_t = "unsigned long" if batch * max(Sq, Sk) * max(D, Dv) >= 2**31 else "unsigned int"
@@ -580,7 +587,8 @@ def _split_tile_lines(nq: int, batch: int, NS: int, KB: int, idx_t: str) -> list
                     f"  const unsigned int sp = (unsigned int)(vh % {NS}u), kb0 = {kb0};"]
 
 
-def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
+def gen_attention(k: Kernel, idx: int, alone: bool = True) -> tuple[str, "Launch"]:  # noqa: F821
+    """``alone``: the kernel is the whole program (``_host_us``)."""
     from .hip_kernels import Launch
 
     q, kk, v = k.inputs
@@ -615,7 +623,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
     if few_queries(Sq):
         bdims = "x".join(str(d) for d in qb_dims) or "1"
         return _gen_few_queries(f"tj{idx}_attention_{bdims}x{Sq}x{Sk}x{D}_{dt.value}_flash", dt, batch, Sq, Sk, D, Dv, scale,
-                                (qoff, qst), (koff, kst), (voff, vst), (ooff, ost))
+                                (qoff, qst), (koff, kst), (voff, vst), (ooff, ost), alone)
     NW, QT = attention_layout(batch, Sq, D, Dv)
     assert QT == 1, "one query tile per wave"
     THREADS = NW * 64
@@ -625,7 +633,7 @@ def gen_attention(k: Kernel, idx: int) -> tuple[str, "Launch"]:  # noqa: F821
     BQ = BQ_PER_WAVE * QT * NW
     KB = -(-Sk // BKV)
     nq = -(-Sq // BQ)
-    NS = key_splits(batch * nq, KB, pingpong, D + Dv, batch * Sq * Dv)
+    NS = key_splits(batch * nq, KB, pingpong, D + Dv, batch * Sq * Dv, alone)
     KBL = -(-KB // NS)                          # key blocks per workgroup
     long = KB - NS * (KBL - 1)                  # splits of KBL blocks; the others have one less
     uneven = long < NS

@@ -106,8 +106,9 @@ def reject_zero_size(nodes) -> None:
             raise NotImplementedError(f"{n.name}: zero-size tensor {tuple(n.shape)} is not supported by the hip backend")
 
 
-def generate_kernel(k: Kernel, idx: int, cfg: MatmulConfig | None = None) -> tuple[str, Launch | list[Launch]]:
-    """HIP source of one fused kernel and its launch(es).  A GEMM whose K is split
+def generate_kernel(k: Kernel, idx: int, cfg: MatmulConfig | None = None,
+                    alone: bool = True) -> tuple[str, Launch | list[Launch]]:
+    """HIP source of one fused kernel (``alone``: the only one of its program) and its launch(es).  A GEMM whose K is split
     across workgroups (``KSPLIT``) writes partial products into a workspace and sums
     them, with the fused epilogue, in each output tile's last workgroup; the M <= 32
     decode kernel (and ``TENSORJIT_HIP_KSPLIT_FUSED=0``) sums them in a second launch."""
@@ -125,7 +126,7 @@ def generate_kernel(k: Kernel, idx: int, cfg: MatmulConfig | None = None) -> tup
     if k.kind == "matmul":
         return gen_matmul(g, cfg or analytic_config(k))
     if k.kind == "attention":
-        return gen_attention(k, idx)
+        return gen_attention(k, idx, alone)
     if k.kind == "colreduce":
         return gen_colreduce(g)
     raise NotImplementedError(k.kind)
@@ -137,7 +138,7 @@ def generate(program: Program, configs: dict[int, MatmulConfig] | None = None) -
     configs = configs or {}
     sources, launches = [PRELUDE], []
     for idx, k in enumerate(program.kernels):
-        src, ls = generate_kernel(k, idx, configs.get(idx))
+        src, ls = generate_kernel(k, idx, configs.get(idx), len(program.kernels) == 1)
         sources.append(src)
         for launch in ls if isinstance(ls, list) else [ls]:
             launch.meta["kernel"] = idx
