@@ -404,7 +404,8 @@ def few_query_splits(batch: int, Sk: int, D: int, Dv: int, alone: bool = True) -
     splits add a combine launch.  Measured: 320 heads x 3000 keys x 128 89.5 us in one part, 77.7
     in two, 75.4 in three (the fuller grid evens out the CUs); 512 heads x 4000 keys 152.8 in
     one, 155.3 in two; 8 heads x 8192 keys 53.2 in one, 10.5 in 16.  ``alone``: see
-    ``_host_us``; at equal calls the count of the shorter kernel."""
+    ``_host_us``; at equal calls the count of the shorter kernel.  A part costs the combine launch
+    about 0.06 us (16 heads x 4096 keys x 64 in a graph 6.3 in 16 parts, 7.6 in 32)."""
     forced = os.environ.get("TENSORJIT_HIP_ATTENTION_SPLITS", "")
     blocks = -(-Sk // FEW_BLOCK)
     if forced.isdigit():
@@ -417,7 +418,7 @@ def few_query_splits(batch: int, Sk: int, D: int, Dv: int, alone: bool = True) -
         resident = min(groups, slots)
         rate = 7e6 * resident / (resident + 75)     # bytes per us: 5.7 TB/s at 320 workgroups
         stream_us = groups * steps * 4 * FEW_BLOCK * (D + Dv) * 2 / rate
-        kernel_us = max(stream_us, -(-groups // slots) * steps * step_us) + (2.5 + 0.02 * n if n > 1 else 0.0)
+        kernel_us = max(stream_us, -(-groups // slots) * steps * step_us) + (2.5 + 0.06 * n if n > 1 else 0.0)
         return max(kernel_us, _host_us(n, alone)), kernel_us
 
     return min((n for n in range(1, 33) if n == 1 or blocks >= 4 * n), key=cost)
@@ -567,7 +568,7 @@ def _gen_few_queries(fname: str, dt: DType, batch: int, Sq: int, Sk: int, D: int
     if NS == 1:
         return src, main
     meta["workspace"] = (ml_base + NS * batch * Sq * 2) * 4
-    meta["ws_arg"] = True
+    meta["ws_arg"] = meta["per_stream"] = True
     combine = gen_combine(fname, dt, batch, Sq, Dv, NS, ooff, ost, idx_t)
     return src + "\n\n" + combine[0], [main, combine[1]]
 
@@ -1389,7 +1390,7 @@ def gen_attention(k: Kernel, idx: int, alone: bool = True) -> tuple[str, "Launch
     if NS == 1:
         return (QUAD_HELPERS if mi16 else "") + "\n".join(L), main
     meta["workspace"] = (ml_base + NS * batch * Sq * 2) * 4
-    meta["ws_arg"] = True
+    meta["ws_arg"] = meta["per_stream"] = True
     combine = gen_combine(fname, dt, batch, Sq, Dv, NS, ooff, ost, idx_t)
     return "\n".join(L) + "\n\n" + combine[0], [main, combine[1]]
 
@@ -1441,6 +1442,6 @@ def gen_combine(fname: str, dt: DType, batch: int, Sq: int, Dv: int, NS: int, oo
          "  }",
          f"  *(tj_u32x4*)&Ob[qrow * {ost}u + d8] = pk;",
          "}"]
-    cmeta = {"family": "attention_combine", "splits": NS, "ws_arg": True, "batch": batch, "Sq": Sq, "Dv": Dv}
+    cmeta = {"family": "attention_combine", "splits": NS, "ws_arg": True, "per_stream": True, "batch": batch, "Sq": Sq, "Dv": Dv}
     comb = Launch(cname, (-(-runs // 256), 1, 1), (256, 1, 1), 0, cmeta)
     return "\n".join(C), comb

@@ -150,14 +150,14 @@ WS_ALIGN = 256
 
 
 def workspace_layout(launches: list[Launch], base: int) -> tuple[dict[int, tuple[int, int]], int]:
-    """Arena ``(offset, bytes)`` of each kernel's workspace (split-K partials), placed
-    after the planned intermediates (``base`` bytes) in the same allocation, and the
-    total arena size."""
+    """Arena ``(offset, bytes)`` of each kernel's workspace (partials that a second launch
+    combines, but for attention's), placed after the planned intermediates (``base`` bytes) in
+    the same allocation, and the total arena size."""
     off = -(-base // WS_ALIGN) * WS_ALIGN
     ws: dict[int, tuple[int, int]] = {}
     for launch in launches:
         need = launch.meta.get("workspace", 0)
-        if need:
+        if need and not launch.meta.get("per_stream"):
             ws[launch.meta["kernel"]] = (off, need)
             off += -(-need // WS_ALIGN) * WS_ALIGN
     return ws, (off if ws else base)
@@ -168,17 +168,21 @@ def launch_args(launches: list[Launch], kernel_args: list[list], ws: dict[int, t
     the launches that take one (``meta["ws_arg"]``) as ``(ARENA, offset, bytes)``.  Products
     split over K (``meta["split_ws"] = (counter bytes, partial bytes)``) use the program's
     per-stream workspace: counters first, partials behind the most counters any launch has
-    (every launch leaves its counters at zero, so launches share both)."""
+    (every launch leaves its counters at zero, so launches share both).  Attention's partials
+    lie there too: whether it splits depends on its sizes, and calls on several streams may not."""
     out = []
     counters = max((l.meta["split_ws"][0] for l in launches if "split_ws" in l.meta), default=0)
-    part0 = -(-counters // WS_ALIGN) * WS_ALIGN
+    part0 = max(1, -(-counters // WS_ALIGN)) * WS_ALIGN
+    rows = {l.meta["kernel"]: l.meta["workspace"] for l in launches if l.meta.get("per_stream") and "workspace" in l.meta}
     for launch in launches:
         idx = launch.meta["kernel"]
         refs = list(kernel_args[idx])
         if "split_ws" in launch.meta:
             cnt, part = launch.meta["split_ws"]
             refs += [(rt.WORKSPACE, 0, cnt), (rt.WORKSPACE, part0, part)]
-        if launch.meta.get("ws_arg"):
+        if launch.meta.get("per_stream"):
+            refs.append((rt.WORKSPACE, part0, rows[idx]))
+        elif launch.meta.get("ws_arg"):
             refs.append((rt.ARENA, *ws[idx]))
         out.append(refs)
     return out
@@ -510,7 +514,9 @@ class HipProgram:
                 self.matmul_configs[idx] = self._pick_config(k, idx, tune)
         self.source, self.launches = generate(program, self.matmul_configs)
         self.code = compile_source(self.source, self.arch, target=self.target)
-        self._workspace, self.arena_bytes = workspace_layout(self.launches, self.plan.arena_bytes)
+        self._workspace, self._arena = workspace_layout(self.launches, self.plan.arena_bytes)
+        # intermediates and the partials of two-launch kernels (attention's are not in the arena)
+        self.arena_bytes = self._arena + sum(l.meta.get("workspace", 0) for l in self.launches if l.meta.get("per_stream"))
         self._native = self._load(self.code, self.launches, launch_args(self.launches, self._args, self._workspace))
 
         self.pool = BufferPool()
@@ -536,7 +542,7 @@ class HipProgram:
     def _load(self, code: bytes, launches: list[Launch], args) -> rt.NativeHipProgram:
         return rt.NativeHipProgram(self.device_index, code, [l.name for l in launches],
                                    [(l.grid, l.block, l.shared) for l in launches], args,
-                                   self.arena_bytes, len(self.program.graph.inputs), len(self._out_nodes))
+                                   self._arena, len(self.program.graph.inputs), len(self._out_nodes))
 
     def _pick_config(self, k: Kernel, idx: int, tune: bool) -> MatmulConfig:
         store = AutotuneStore()

@@ -42,6 +42,19 @@ def test_seventeen_queries_and_a_forced_schedule_keep_the_tiled_kernels(monkeypa
     assert launches_of(shapes(1))[1][0].meta["schedule"] == "double-buffer"
 
 
+def test_partials_lie_in_the_streams_workspace():
+    """Both launches of a split call, few queries and tiled, get the same per-stream memory."""
+    from tensorjit.runtime import hip as rt
+    for shapes in ([(320, n, 64) for n in (1, 1500, 1500)], [(8, n, 128) for n in (500, 1450, 1450)]):
+        _, launches = launches_of(shapes)
+        for launch in launches:
+            launch.meta["kernel"] = 0
+        layout, arena = hb.workspace_layout(launches, 512)
+        refs = hb.launch_args(launches, [[]], layout)
+        assert arena == 512 and not layout
+        assert refs[0] == refs[1] == [(rt.WORKSPACE, hb.WS_ALIGN, launches[0].meta["workspace"])]
+
+
 def test_every_split_has_a_block():
     for batch in (1, 3, 8, 100, 320, 512, 5000):
         for Sk in (1, 31, 32, 33, 127, 1000, 1025, 4000, 8191):

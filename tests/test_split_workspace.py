@@ -74,6 +74,27 @@ def test_graphs_of_one_program_and_eager_calls_overlap():
     assert prog.stats()["workspace_blocks"] == 3
 
 
+@pytest.mark.parametrize("heads,Sq,Sk,D", [(320, 1, 1500, 64), (8, 500, 1450, 128)])
+def test_key_split_attention_on_several_streams(heads, Sq, Sk, D):
+    """A lone attention call, split over its keys by a rule on its sizes, on three streams
+    without any ordering between them: bit-equal to calls one after the other."""
+    fn = tj.jit(lambda q, k, v: tj.matmul(tj.softmax(tj.matmul(q, tj.transpose(k, -1, -2)) * D ** -0.5), v), tune=False)
+    gen = torch.Generator(device=DEV).manual_seed(heads)
+    cases = [[torch.randn(heads, n, D, device=DEV, generator=gen).half() for n in (Sq, Sk, Sk)] for _ in range(3)]
+    cp = fn.compiled(*cases[0])
+    assert cp.launches[0].meta["splits"] > 1 and cp.native.arena()[1] == 0
+    refs = [fn(*c).clone() for c in cases]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in cases]
+    got = [[] for _ in cases]
+    for _ in range(10):
+        for s, c, g in zip(streams, cases, got):
+            with torch.cuda.stream(s):
+                g.append(fn(*c))
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, ref) for ref, g in zip(refs, got) for o in g)
+
+
 def test_first_call_on_a_stream_returns_while_the_stream_is_busy():
     prog, args, ref, out = _split_program()
     prog.run(*_ptrs(args, out), _stream())               # the block allocated with the program is taken
