@@ -37,7 +37,7 @@ from ..runtime.autotune import MatmulConfig
 from .common import access_strides, contiguous_strides, emit_expr
 from .hip_kernels import KernelGen, Launch
 from .hip_prelude import CTYPE
-from .hip_ring import ring_epilogue_lines, ring_fits, ring_loop_lines, ring_ok, ring_split_lines
+from .hip_ring import WAVE_SYNC, ring_epilogue_lines, ring_fits, ring_loop_lines, ring_ok, ring_split_lines
 
 # (dtype, MI) -> (builtin, KI = K per instruction, KPL = K elements per lane, acc regs, operand vector type)
 MFMA = {
@@ -525,8 +525,10 @@ def direct_staged_epilogue_lines(g, k, mm, epilogue, epi_inputs, out_shape, bidx
     owns array w and stages its sub-tile through it 32 rows (one 32x32 or two 16x16
     MFMA row blocks) at a time, with no further workgroup barriers: a wave's LDS
     accesses complete in order.  Each pass turns the MFMA layout into 16-byte runs of
-    output rows, as in the shared staged epilogue.  Returns None where the arrays do
-    not fit a pass."""
+    output rows, as in the shared staged epilogue.  Its lanes read what others wrote, so where
+    a condition splits them (edges of M and N) wave barriers keep the compiler from taking
+    some of them on to the next pass's writes first.  Returns None where the arrays do not fit
+    a pass."""
     out_dt = k.outputs[0].dtype
     if cfg.num_warps != 4 or any(o.dtype != out_dt for o in k.outputs):
         return None
@@ -540,7 +542,9 @@ def direct_staged_epilogue_lines(g, k, mm, epilogue, epi_inputs, out_shape, bidx
     L = ["  __syncthreads();",
          "  float* Cw = (float*)(wave == 0u ? As0 : wave == 1u ? As1 : wave == 2u ? Bs0 : Bs1);"]
     tiles = 32 // MI                      # MFMA row blocks per 32-row pass
+    sync = [WAVE_SYNC] if guard_m or guard_n or 32 * per_row % 64 else []
     for p_ in range(TMW // tiles):
+        L += sync if p_ else []
         for xl in range(tiles):
             x = p_ * tiles + xl
             row = ("(r / 4) * 8 + (lane / 32u) * 4 + (r % 4)" if MI == 32
@@ -550,6 +554,7 @@ def direct_staged_epilogue_lines(g, k, mm, epilogue, epi_inputs, out_shape, bidx
             L.append("#pragma unroll")
             L.append(f"  for (int r = 0; r < {NACC}; ++r)")
             L.append(f"    Cw[({row}) * {ldc}u + y * {MI}u + lane % {MI}u] = acc[{x}][y][r];")
+        L += sync
         L.append("#pragma unroll")
         L.append(f"  for (unsigned int c = lane; c < {32 * per_row}u; c += 64u) {{")
         L.append(f"    const unsigned int lr = c / {per_row}u, cc = (c % {per_row}u) * {ve}u;")

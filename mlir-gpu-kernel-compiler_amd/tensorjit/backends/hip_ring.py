@@ -32,6 +32,7 @@ from ..ir import DType
 
 OOB = "0x80000000u"      # a byte offset past every descriptor's range: the load returns zeros
 NW_MAX_VMCNT = 63
+WAVE_SYNC = '  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier();'
 
 
 def ring_ok(cfg, dt: DType) -> bool:
@@ -307,7 +308,7 @@ def ring_epilogue_lines(cfg, out_dts, N: int, M: int, guard_m: bool, guard_n: bo
     # lanes exchange values through Cw within a wave: the wave barriers keep the compiler from
     # running one branch of a divergent condition (few runs per row, tile edges) through
     # several blocks before the other lanes' branch
-    sync = ['  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier();']
+    sync = [WAVE_SYNC]
     L = ["  __syncthreads();", f"  float* Cw = (float*)({sel});"]
     for x in range(TMW):
         L += sync if x else []

@@ -39,8 +39,11 @@ DIRECT = MatmulConfig(256, 256, 64, 4, 2, 2, 32, 1, 8, 0, 0, 1)
 DIRECT_N128 = MatmulConfig(256, 128, 64, 4, 2, 2, 32, 1, 8, 0, 0, 1)
 DIRECT16 = MatmulConfig(256, 256, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1)
 DIRECT16_N128 = MatmulConfig(256, 128, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1)
-ALL_DIRECT = [DIRECT, DIRECT_N128, DIRECT16, DIRECT16_N128]
-DIRECT_IDS = ["256x256", "256x128", "256x256_mi16", "256x128_mi16"]
+# 96 rows or columns per wave
+WIDE16 = [MatmulConfig(m, n, 64, 4, 2, 2, 16, 1, 8, 0, 0, 1)
+          for m, n in ((256, 192), (192, 256), (192, 192), (192, 128), (128, 192))]
+ALL_DIRECT = [DIRECT, DIRECT_N128, DIRECT16, DIRECT16_N128, *WIDE16]
+DIRECT_IDS = ["256x256", "256x128", "256x256_mi16", "256x128_mi16", *(f"{c.TM}x{c.TN}_mi16" for c in WIDE16)]
 # fp32 operands: 32-deep K tiles (the same 128-byte rows), 16x16x4 MFMAs
 F32_DIRECT = [MatmulConfig(128, 128, 32, 4, 2, 2, 16, 1, 8, 0, 0, 1), MatmulConfig(256, 128, 32, 4, 2, 2, 16, 1, 8, 0, 0, 1),
               MatmulConfig(128, 256, 32, 4, 2, 2, 16, 1, 8, 0, 0, 1), MatmulConfig(64, 64, 32, 4, 2, 2, 16, 1, 8, 0, 0, 1)]
@@ -151,6 +154,22 @@ def test_direct_kernels_compile_for_gfx950(epi, shape, tj_env):
         assert launches[0].meta.get("epilogue") == "lds-staged"
         assert "raw_ptr_buffer_load_lds" in src and "__builtin_amdgcn_s_waitcnt(0x0F70);" in src
         hb.compile_source(src, "gfx950")
+
+
+@pytest.mark.parametrize("cfg", ALL_DIRECT, ids=DIRECT_IDS)
+def test_staged_epilogue_passes_are_ordered_where_lanes_part(cfg):
+    """Each pass writes LDS, reads what other lanes wrote and skips what is past M and N: a wave
+    barrier stands between its writes and its reads, and before the next pass's writes.  (Whole
+    tiles have no condition that lanes could part at.)"""
+    sync = "__builtin_amdgcn_wave_barrier();"
+    for shape, parts in (((300, 520, 192), True), ((2 * cfg.TM, 2 * cfg.TN, 64), False)):
+        src, _ = _source(cfg, *shape)
+        epi = src[src.index("  float* Cw = "):]
+        events = re.findall(r"(    Cw\[.*\] = acc)|(= tj_.*Cw\[|[^\n]*Cw\[lr)|(" + re.escape(sync) + ")", epi)
+        kinds = "".join("w" if w else "r" if r else "s" for w, r, _ in events)
+        passes = cfg.TM // cfg.WM // 32
+        one = "w" * (32 // cfg.MI)
+        assert re.sub("r+", "r", kinds) == ("s".join([one + "sr"] * passes) if parts else (one + "r") * passes), kinds
 
 
 def test_direct_config_rules():
