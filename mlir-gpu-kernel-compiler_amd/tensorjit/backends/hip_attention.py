@@ -880,7 +880,8 @@ def gen_attention(k: Kernel, idx: int, alone: bool = True) -> tuple[str, "Launch
         if mi16:
             return block_max16(sc, j, pre)
         mask = None
-        if ragged and (j == KBL - 1 or uneven and j == KBL - 2):
+        # the block cut by Sk is the last of the last split, which is a short one of uneven splits
+        if ragged and j == KBL - (2 if uneven else 1):
             mask = f"{j * BKV}" if NS == 1 else f"(int)kb0 * {BKV} + {j * BKV}"
         elif ragged and j is None and pingpong:
             mask = "(int)jj"

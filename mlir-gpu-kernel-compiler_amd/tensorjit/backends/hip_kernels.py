@@ -214,7 +214,7 @@ def gen_pointwise(g: KernelGen, nodes: list[Node], iter_shape: tuple[int, ...]) 
     # was bound by the count of its loads: the two-input gelu / sigmoid chain with row-broadcast
     # scale and shift (one box, us) bf16 [16384, 4095] 150.7 -> 68.7 (5.9 TB/s), [50000, 301]
     # 27.3 -> 17.4, fp32 [16384, 4095] 172.3 -> 131.5.
-    ragged = vec == 1 and vec_width(dt) <= row_len and row_len * 2 > vec_width(dt) and iter_shape != ()
+    ragged = vec == 1 and vec_width(dt) <= row_len and iter_shape != ()
     if ragged:
         vec = vec_width(dt)
         vpr = -(-row_len // vec)

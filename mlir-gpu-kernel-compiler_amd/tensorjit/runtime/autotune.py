@@ -6,16 +6,17 @@ best ``top_k`` are compiled and timed on real buffers, and the winner is
 persisted in ``AutotuneStore`` so later processes start warm.
 
 The model is re-derived for MI355X instead of the reference's GPU branch
-(``autotune.py:73-79``).  It prices one call as the slowest of
+(``autotune.py:73-79``): times fitted to measurements for the ring, direct-to-LDS and decode
+schedules, and for register-staged tiles the slowest of
 
 * MFMA time: 2*M*N*K at the dense matrix-core peak, scaled by how well the
   tile grid fills 256 CUs (tail rounds of workgroups) and by edge waste;
 * LDS time: every wave re-reads its A and B fragments from LDS each K step
   (128 B/clk/CU);
 * L2 time: each workgroup streams a (BM + BN) x K panel;
-* HBM time: A, B and C once at 8 TB/s;
+* HBM time: A, B and C once at 8 TB/s.
 
-and rejects tiles that exceed 160 KiB of double-buffered LDS or 512 VGPRs
+It rejects staged tiles that exceed 160 KiB of double-buffered LDS or 512 VGPRs
 (accumulators + fragments + staging) per lane.
 """
 from __future__ import annotations
@@ -178,7 +179,7 @@ def ring_candidates(M: int, N: int, K: int, batch: int, itemsize: int) -> list[M
     return out
 
 
-# (TM, TN, waves, WM, WN, STAGES): what 64 KiB - 144 KiB of LDS hold.  Of these the small tiles
+# (TM, TN, waves, WM, WN, STAGES): 32 KiB (32x32) to 128 KiB (128x128) of LDS.  Of these the small tiles
 # win while the grid leaves CUs idle, 128x128 with 8 waves (two per SIMD, one workgroup per CU)
 # once it is full.
 RING_TILES = [
@@ -211,7 +212,6 @@ def _ring_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
     t_mfma = w * per * mflop
     t_dma = w * per * (tm + tn) * 0.128 * 0.0085
     t_lat = rounds * per * 0.1 / (cfg.STAGES - 1) ** 0.89
-    # weights of up to ~64 MB come from the MALL on a repeated call; more stream from HBM
     mem = _hbm_us(M, N, K, batch, elem, mats)
     t_hbm = mem / 9.42
     edge = 4.0 if N % (16 // elem) else 1.0                       # element-wise stores of ragged rows
@@ -319,15 +319,8 @@ def _skinny_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: in
 
 
 def _sched_factor(cfg: MatmulConfig) -> float:
-    """Relative MFMA-phase cost of a loop schedule, from bf16 8192^3 runs on MI355X
-    (direct-to-LDS loads 3-7% ahead of ping-pong with K-split tiles, and another ~10%
-    with 16x16x32 MFMAs, which hold a higher clock on random data than 32x32x16;
-    plain double-buffered loop ~9% behind ping-pong; the persistent direct kernel
-    1-2% ahead of the direct one at 8192^3, 1-8% on config 5's projections)."""
-    if cfg.PERSIST:
-        return 0.85
-    if cfg.DIRECT:
-        return 0.86 if cfg.MI == 16 else 0.95
+    """Relative MFMA-phase cost of a register-staged loop schedule, from bf16 NT 8192^3 runs on
+    MI355X (the plain double-buffered loop ~9% behind ping-pong with K-split tiles)."""
     if cfg.INTERLEAVE:
         return 1.15
     return {3: 1.0, 2: 1.04, 1: 1.05}.get(cfg.PINGPONG, 1.09)
@@ -343,17 +336,15 @@ def _hip_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
         return _direct_cost(cfg, M, N, K, batch, elem, mats)
     tm, tn, tk = cfg.TM, cfg.TN, cfg.TK or 32
     waves = cfg.num_warps
-    if cfg.SPLIT_K == 1 and (tm % (cfg.WM * cfg.MI) or tn % (cfg.WN * cfg.MI)):
+    if tm % (cfg.WM * cfg.MI) or tn % (cfg.WN * cfg.MI):
         return math.inf
     pad = 16 // elem
     lds = 2 * (tm + tn) * (tk + pad) * elem
     if lds > LDS_BYTES_PER_CU:
         return math.inf
-    acc = tm * tn / (64 * waves) * (cfg.SPLIT_K if cfg.SPLIT_K > 1 else 1)
+    acc = tm * tn / (64 * waves)
     frags = 2 * (tm / cfg.WM + tn / cfg.WN) / cfg.MI * (4 if elem == 2 else 1)  # double-buffered
-    if cfg.DIRECT and cfg.MI == 16:
-        frags -= tm / cfg.WM / cfg.MI * 4                                   # A re-read in place
-    staging = 0 if cfg.DIRECT else (tm + tn) * tk * elem / (64 * waves * 4)  # staged K step per lane, 4 B per VGPR
+    staging = (tm + tn) * tk * elem / (64 * waves * 4)                      # staged K step per lane, 4 B per VGPR
     regs = acc + frags + staging + 32
     if regs > 512:
         return math.inf
@@ -377,12 +368,8 @@ def _hip_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
     t_l2 = tiles * (tm + tn) * kt * elem / L2_BYTES_PER_S
     t_hbm = (M * K + N * K + M * N) * batch * elem / HBM_BYTES_PER_S
     # a workgroup writes its output tile after its K loop; with one workgroup per CU
-    # nothing overlaps that store, which matters when the output dominates (small K);
-    # a persistent workgroup starts its next tile while the stores drain (about half
-    # of them overlap: the second K step of the next tile waits for them)
+    # nothing overlaps that store, which matters when the output dominates (small K)
     t_out = M * N * batch * (4 * S if S > 1 else elem) / HBM_BYTES_PER_S / occ
-    if cfg.PERSIST and tiles > CU_COUNT:
-        t_out *= 0.5
     # split K: the S fp32 partials are read back and the output written after the last
     # split finishes (in the tile's last workgroup, ~2.3 us of tail at config 1, or a second launch)
     t_sum = ((S * 4 + elem) * M * N * batch / HBM_BYTES_PER_S + 4e-6) if S > 1 else 0.0
