@@ -195,6 +195,9 @@ POINTWISE_UNROLL = 1
 POINTWISE_THREADS = 128
 
 
+RAGGED_POINTWISE_BYTES = 1 << 20
+
+
 def gen_pointwise(g: KernelGen, nodes: list[Node], iter_shape: tuple[int, ...]) -> tuple[str, Launch]:
     """Fused pointwise DAG ``nodes`` over ``iter_shape`` (elementwise kernels and
     reduction-free row groups)."""
@@ -213,8 +216,12 @@ def gen_pointwise(g: KernelGen, nodes: list[Node], iter_shape: tuple[int, ...]) 
     # neighbour are computed twice, from the same inputs to the same bits.  One element per lane
     # was bound by the count of its loads: the two-input gelu / sigmoid chain with row-broadcast
     # scale and shift (one box, us) bf16 [16384, 4095] 150.7 -> 68.7 (5.9 TB/s), [50000, 301]
-    # 27.3 -> 17.4, fp32 [16384, 4095] 172.3 -> 131.5.
-    ragged = vec == 1 and vec_width(dt) <= row_len and iter_shape != ()
+    # 27.3 -> 17.4, fp32 [16384, 4095] 172.3 -> 131.5.  Below a MB a launch is all latency, which
+    # the row and column of every vector lengthen (65 random shapes in all dtypes, mean: elements
+    # 3.03, vectors 3.21; the 14 of 100 KB to 1 MB 3.04, 3.33).  From 1.3 MB vectors are always
+    # ahead (25 shapes; fp16 [324, 2074] 3.7 / 3.3, [197629, 10] 6.1 / 3.5).
+    ragged = (vec == 1 and vec_width(dt) <= row_len and iter_shape != ()
+              and numel * dt.itemsize >= RAGGED_POINTWISE_BYTES)
     if ragged:
         vec = vec_width(dt)
         vpr = -(-row_len // vec)
