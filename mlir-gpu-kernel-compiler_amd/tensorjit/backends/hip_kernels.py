@@ -953,9 +953,16 @@ def col_workgroups_per_cu(streamed_bytes: int) -> int:
     return 4
 
 
-def col_layout(A: int, Rd: int, B: int, vec: int, streamed_bytes: int = 0) -> tuple[int, int, int]:
+def col_layout(A: int, Rd: int, B: int, vec: int, streamed_bytes: int = 0, few: bool = False,
+               itemsize: int = 4) -> tuple[int, int, int]:
     """(column blocks per A-slice nb, rows per workgroup RS, splits S) of a column reduction
-    whose inputs stream ``streamed_bytes``."""
+    whose inputs stream ``streamed_bytes``.  ``few``: rows of unaligned vectors, which have a
+    quarter or an eighth of the column blocks that one element per lane has; the splits that
+    fill the same workgroups with them cost the combine launch more than they give.  us, splits
+    as many / fewer: bf16 [12769, 498] 511 8.8 / 256 6.7 (one element per lane 7.3), [3, 4286,
+    445] 253 8.2 / 127 7.1 (7.0), [9692, 316] 511 8.4 / 256 6.5 (6.1), fp32 [29, 43, 2893] 2 5.9
+    / 1 4.0 (4.3).  fp32 sums keep their longer splits where there is more than that to walk:
+    shorter ones are the more exact."""
     L = -(-B // vec)
     nb = -(-L // 64)
     base = A * nb
@@ -965,6 +972,10 @@ def col_layout(A: int, Rd: int, B: int, vec: int, streamed_bytes: int = 0) -> tu
     else:
         wgs = col_workgroups_per_cu(streamed_bytes) * CU_COUNT
         S = max(1, min(-(-wgs // base), Rd // COL_MIN_ROWS, COL_MAX_SPLITS))
+        if few and itemsize < 4:
+            S = max(1, min(S, 384 // base, CU_COUNT))
+        elif few and base >= CU_COUNT and Rd < 4 * COL_MIN_ROWS:
+            S = 1
     RS = -(-Rd // S)
     return nb, RS, -(-Rd // RS)
 
@@ -993,7 +1004,7 @@ def gen_colreduce(g: KernelGen) -> tuple[str, Launch | list[Launch]]:
         vec = vec_width(dt)
     streamed = sum(math.prod(n.shape) * n.dtype.itemsize for n in xin if _streamed(Sx, xstr[id(n)]))
     nt = _nt_loads(streamed)
-    nb, RS, S = col_layout(A, Rd, B, vec, streamed)
+    nb, RS, S = col_layout(A, Rd, B, vec, streamed, ragged, dt.itemsize)
     L = -(-B // vec)
     AB = A * B
     idx_t = _index_type(A * Rd * B)
@@ -1004,7 +1015,7 @@ def gen_colreduce(g: KernelGen) -> tuple[str, Launch | list[Launch]]:
 
     narrow = A == 1 and B * dt.itemsize < COL_NARROW_BYTES
     if narrow:
-        S, RS = col_narrow_layout(Rd, L, streamed)
+        S, RS = col_narrow_layout(Rd, L, streamed, dt.itemsize)
 
     def fold(acc: str, v: str) -> str:
         return f"{acc} = fmaxf({acc}, {v});" if is_max else f"{acc} += {v};"
@@ -1121,9 +1132,16 @@ COL_NARROW_BYTES = 512
 COL_NARROW_LANES = 256
 
 
-def col_narrow_layout(Rd: int, L: int, streamed_bytes: int) -> tuple[int, int]:
+def col_narrow_layout(Rd: int, L: int, streamed_bytes: int, itemsize: int = 4) -> tuple[int, int]:
     """(workgroups S, rows per workgroup) of a narrow column reduction: four workgroups per CU
-    or fewer, four rows per lane group at least."""
+    or fewer, four rows per lane group at least.
+
+    Every workgroup counts itself in one counter, so many of them cost more than they read.
+    us at S: bf16 [25133, 58] 195 8.0, 98 5.9 (one element per lane 6.6), fp16 [395258, 10] 512
+    12.1, 128 7.2 (10.1), [950360, 9] 512 14.1, 128 12.7, bf16 [6109, 172] 136 10.8, 64 6.0,
+    [618418, 72] 448 25.1, 128 19.6; and a walk of 32 rows is shorter than any counting:
+    [1141, 9] 2 5.6, 1 4.0 (4.5), [4035, 12] 7 5.6, 1 5.1 (5.0).  fp32 keeps more and shorter
+    sums: they are the more exact."""
     G = COL_NARROW_LANES // L
     forced = os.environ.get("TENSORJIT_HIP_COL_SPLITS")
     if forced and forced.isdigit():
@@ -1132,6 +1150,8 @@ def col_narrow_layout(Rd: int, L: int, streamed_bytes: int) -> tuple[int, int]:
         # at most 16 partials per lane group for the finishing workgroup (bf16 [20000, 255], 8
         # groups: 512 workgroups 61 us, 128 8.5)
         S = max(1, min(col_workgroups_per_cu(streamed_bytes) * CU_COUNT, Rd // (4 * G), 16 * G, COL_MAX_SPLITS))
+        if itemsize < 4:
+            S = 1 if Rd <= 32 * G else min(S, max(64, Rd // (8 * G)), 128)
     RS = -(-Rd // S)
     return -(-Rd // RS), RS
 

@@ -7,6 +7,7 @@ import tensorjit as tj
 from parity import close_f32, close_lowp
 from tensorjit import compiler as C
 from tensorjit.backends import hip_backend as hb
+from tensorjit.backends import hip_kernels as hk
 from tensorjit.ir import DType, TensorType
 
 DEV = "cuda:0"
@@ -21,6 +22,23 @@ def test_pointwise_rows_take_unaligned_vectors_from_a_megabyte(dt):
         p = C.lower(tj.trace(lambda x, b: x + b, [TensorType((rows, n), dt), TensorType((n,), dt)]), "hip")
         _, (launch,) = hb.generate(p)
         assert launch.meta["family"] == "pointwise" and launch.meta["unaligned"] == unaligned
+
+
+@pytest.mark.parametrize("itemsize", [2, 4])
+@pytest.mark.parametrize("Rd,B", [(1, 9), (1141, 9), (4096, 9), (4097, 9), (6109, 172), (25133, 58), (395258, 10), (1 << 20, 4)])
+def test_narrow_columns_split_few_times_and_cover_every_row(Rd, B, itemsize):
+    L = -(-B // (16 // itemsize))
+    S, RS = hk.col_narrow_layout(Rd, L, Rd * B * itemsize, itemsize)
+    assert (S - 1) * RS < Rd <= S * RS
+    if itemsize == 2:
+        assert S <= 128 and (S == 1) == (Rd <= 32 * (256 // L))
+
+
+def test_unaligned_wide_columns_split_fewer_times():
+    for A, Rd, B, most in [(1, 12769, 498, 256), (3, 4286, 445, 128), (1, 9692, 316, 256)]:
+        nb, RS, S = hk.col_layout(A, Rd, B, 8, 0, few=True, itemsize=2)
+        assert S <= most < hk.col_layout(A, Rd, B, 8)[2] and (S - 1) * RS < Rd <= S * RS
+    assert hk.col_layout(29, 43, 2893, 4, 0, few=True)[2] == 1 < hk.col_layout(29, 43, 2893, 4)[2]
 
 
 @pytest.mark.gpu
@@ -38,3 +56,15 @@ def test_unaligned_pointwise_matches_float64(dt, rows, n):
     close = close_f32 if dt == torch.float32 else close_lowp
     close(out, X * G + Y * Cc)
     close(s, torch.sigmoid(X))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("shape,axis", [((1141, 9), 0), ((4096, 9), 0), ((4097, 9), 0), ((6109, 172), 0), ((25133, 58), 0),
+                                        ((12769, 498), 0), ((3, 4286, 445), 1), ((29, 43, 2893), 1)])
+def test_columns_are_exact_on_integers(dt, shape, axis):
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randint(-1, 2, shape, device=DEV, generator=gen).to(dt)
+    f = tj.jit(lambda t: tj.sum(t, axis=axis))
+    for _ in range(2):
+        assert torch.equal(f(x), x.double().sum(axis).to(dt))
