@@ -294,6 +294,7 @@ def _staged_us(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, tb: bool) 
     cut = max(cut_m if M % cfg.TM else 1.0, cut_n if N % cfg.TN else 1.0)
     # what the estimate misses: a launch's start, few K steps, output rows off the 128-byte lines
     lead = (1.24 if not tb and N % 64 else 1.0) / (0.93 if K < 256 else 1.0)
+    epi += 13.0 if N % 8 else 0.0                                 # element-wise stores
     return ((rounds - 1 + last) * (-(-K // cfg.TK) * step + epi) * cut + 2.0) * lead
 
 

@@ -84,6 +84,7 @@ def test_ring_candidates_are_valid_and_bounded():
 @pytest.mark.parametrize("m,n,k,tb,lead,staged", [
     (8192, 8192, 8192, False, (), True), (4096, 4096, 16384, False, (), True), (16384, 4096, 4096, False, (), True),
     (512, 512, 512, False, (64,), True), (8192, 8192, 8200, True, (), True), (2048, 11008, 4104, True, (), True),
+    (4096, 4095, 4104, True, (), True),
     (2048, 4096, 4096, False, (), False), (2048, 11008, 4096, False, (), False), (1000, 4096, 4104, True, (), False)])
 def test_products_without_a_direct_tile_keep_the_256_wide_staged_ones(m, n, k, tb, lead, staged):
     """The choice without tuning, and what tuning may time: products of whole rounds of 256x256
@@ -120,6 +121,8 @@ def test_products_with_a_direct_tile_time_no_staged_ones():
     (kernel,) = _program(2048, 4096, 4096, True, DType.bf16).kernels
     assert all(c.STAGES or c.DIRECT or c.SPLIT_K > 1 for c in hb._candidates(kernel))
     (kernel,) = _program(4096, 4096, 4096, False, DType.f32).kernels
+    assert all(c.STAGES for c in hb._candidates(kernel))
+    (kernel,) = _program(700, 1501, 520, True, DType.bf16).kernels      # odd N: stores one by one
     assert all(c.STAGES for c in hb._candidates(kernel))
 
 
