@@ -126,6 +126,15 @@ def test_products_with_a_direct_tile_time_no_staged_ones():
     assert all(c.STAGES for c in hb._candidates(kernel))
 
 
+@pytest.mark.parametrize("m,n,k,direct", [(4096, 4096, 4096, True), (4096, 4096, 512, True), (2048, 4096, 1024, True),
+                                          (512, 3072, 768, False), (512, 768, 3072, False)])
+def test_fp32_products_of_a_full_grid_take_direct_tiles(m, n, k, direct):
+    """Direct-to-LDS tiles measured 3-9% ahead of the ring there, and far behind it short of tiles."""
+    (kernel,) = _program(m, n, k, True, DType.f32).kernels
+    cfg = hb.analytic_config(kernel)
+    assert bool(cfg.DIRECT) == direct and bool(cfg.STAGES) == (not direct), cfg
+
+
 def test_split_launches_share_the_workspace():
     """Counters at the head of the block, as many as any launch has; partials behind them."""
     dt = DType.bf16
