@@ -114,7 +114,9 @@ int tj_hip_program_create(int device, const void* code, size_t code_size, int nk
                           const char* const* names, const tj_launch* launches, const tj_argref* args,
                           size_t arena_bytes, int n_inputs, int n_outputs, void** handle);
 
-/* Launch every kernel in order on `stream` (a hipStream_t; NULL = default stream).
+/* Launch every kernel in order on `stream` (a hipStream_t; NULL = default stream).  Inputs and
+ * outputs must not overlap: kernels may read an input element after its neighbour's lane has
+ * written (all pointers are declared __restrict__).
  * Asynchronous: never waits for `stream`.  A program with a workspace allocates a block the
  * first time it meets a second stream or capture: cleared in order on the stream, under
  * capture on a stream of its own that the call waits for.  A 41st stream waits for the device
