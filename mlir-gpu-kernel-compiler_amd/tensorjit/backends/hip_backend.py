@@ -29,7 +29,7 @@ from ..passes.fusion import _finalize
 from ..passes.memory_planner import MemoryPlan, plan_memory
 from ..runtime import hip as rt
 from ..runtime.autotune import (HIP_CANDIDATES, HIP_F32_CANDIDATES, MatmulConfig, autotune, beside_ring, cost_model,
-                                ring_candidates)
+                                fp32_factor, ring_candidates)
 from ..runtime.cache import AutotuneStore, CodeObjectCache
 from ..runtime.dtypes import TORCH_DTYPE
 from ..runtime.pool import BufferPool
@@ -69,15 +69,16 @@ def _candidates(k: Kernel) -> list[MatmulConfig]:
     return ring + [c for c in cands if c.DIRECT or c.SPLIT_K > 1 or staged and beside_ring(c)]
 
 
-def _rank(k: Kernel, cands: list[MatmulConfig]):
-    """The cost of a tiling of ``k`` among ``cands``."""
+def _rank(k: Kernel, cands: list[MatmulConfig], fitted: bool = True):
+    """The cost of a tiling of ``k`` among ``cands`` (``fitted``: with ``fp32_factor``)."""
     mm = k.anchor
     M, N, K, tb = matmul_dims(mm)
     batch = math.prod(mm.shape[:-2]) if len(mm.shape) > 2 else 1
     kind = "hip_f32" if compute_dtype(mm) == DType.f32 else "hip"
     ring_nt = tb if any(c.STAGES for c in cands) and any(beside_ring(c) for c in cands) else None
     mats = tuple(math.prod(n.shape[:-2]) for n in mm.inputs)
-    return lambda c: cost_model(c, M, N, K, kind, batch, ring_nt, mats)
+    fit = lambda c: fp32_factor(c, M, N, batch) if fitted and kind == "hip_f32" else 1.0  # noqa: E731
+    return lambda c: cost_model(c, M, N, K, kind, batch, ring_nt, mats) * fit(c)
 
 
 def matmul_key(k: Kernel, arch: str) -> str:
@@ -89,8 +90,15 @@ def matmul_key(k: Kernel, arch: str) -> str:
 
 
 def analytic_config(k: Kernel) -> MatmulConfig:
+    """The cheapest tiling.  fp32 products whose unfitted estimates choose a K split keep it (its
+    shorter sums are the more exact); unsplit ones go by the fitted estimates: those of a full grid
+    to the direct-to-LDS tiles (us, ring 128x128 / direct: 4096^3 966 / 908, 4096 x 4096 x 512 134 /
+    122, 5 x 1010 x 5216 x 384 187 / 169)."""
     cands = _candidates(k)
-    return min(cands, key=_rank(k, cands))
+    best = min(cands, key=_rank(k, cands, fitted=False))
+    if compute_dtype(k.anchor) == DType.f32 and best.KSPLIT == 1:
+        best = min([c for c in cands if c.KSPLIT == 1], key=_rank(k, cands))
+    return best
 
 
 # ---------------------------------------------------------------------------

@@ -211,10 +211,7 @@ def _ring_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
     occ = max(1, min(LDS_BYTES_PER_CU // (cfg.STAGES * (tm + tn) * 128 + 64), 32 // cfg.num_warps))
     w = -(-wgs // CU_COUNT)
     rounds, conc = -(-w // occ), min(w, occ)
-    # us per MFLOP of a CU's MFMAs; fp32 tiles of 4 waves two and more to a CU overlap better
-    # (0.83-0.89 of the model without it in 14 shapes)
-    rate = 0.2465 if elem == 2 else 1.72 if wgs >= 2 * CU_COUNT and cfg.num_warps == 4 else 2.04
-    mflop = tm * tn * cfg.TK * 2e-6 * rate * (0.88 if cfg.num_warps == 8 else 1.0)
+    mflop = tm * tn * cfg.TK * 2e-6 * (0.2465 if elem == 2 else 2.04) * (0.88 if cfg.num_warps == 8 else 1.0)
     t_mfma = w * per * mflop
     t_dma = w * per * (tm + tn) * 0.128 * 0.0085
     t_lat = rounds * per * 0.1 / (cfg.STAGES - 1) ** 0.89
@@ -256,11 +253,6 @@ def _direct_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: in
         occ = 1 if cfg.PERSIST else max(1, min(LDS_BYTES_PER_CU // (2 * (tm + tn) * 128), 2))
         mflop = tm * tn * cfg.TK * 2e-6 * (0.14 if elem == 2 else 2.0)
         one, epi = mflop + (tm + tn) * 1e-3 * 0.396, tm * tn * 1e-3 * 0.2156 * occ
-        if elem == 4:
-            # measured at 0.73-0.87 of this (64x64 to 128x256, 15 NT shapes): with it fp32 products
-            # of a full grid stay on these tiles (4096^3 908 us, ring 934-966; 4096 x 4096 x 512
-            # 122, 127-134)
-            one, epi = one * 0.79, epi * 0.79
         full = one * occ
     if cfg.MI == 32:
         one, full = one * 1.1, full * 1.1                         # lower clock on random data
@@ -388,6 +380,16 @@ def _hip_cost(cfg: MatmulConfig, M: int, N: int, K: int, batch: int, elem: int,
     t_sum = ((S * 4 + elem) * M * N * batch / HBM_BYTES_PER_S + 4e-6) if S > 1 else 0.0
     t = max(t_mfma, t_lds, t_l2, t_hbm) + t_out + t_sum
     return t * 1e6
+
+
+def fp32_factor(cfg: MatmulConfig, M: int, N: int, batch: int) -> float:
+    """Measured time of an fp32 tiling of a full grid over its estimate: 0.73-0.87 for the
+    direct-to-LDS tiles (64x64 to 128x256, 15 NT shapes), 0.83-0.89 for the ring's 4-wave tiles
+    two and more to a CU (14 shapes), 1 for its 128x128."""
+    if cfg.DIRECT:
+        return 0.79
+    wgs = -(-M // cfg.TM) * -(-N // cfg.TN) * batch * cfg.KSPLIT
+    return 0.86 if cfg.STAGES and cfg.num_warps == 4 and wgs >= 2 * CU_COUNT else 1.0
 
 
 def cost_model(cfg: MatmulConfig, M: int, N: int, K: int, backend: str, batch: int = 1,

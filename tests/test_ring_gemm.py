@@ -135,6 +135,16 @@ def test_fp32_products_of_a_full_grid_take_direct_tiles(m, n, k, direct):
     assert bool(cfg.DIRECT) == direct and bool(cfg.STAGES) == (not direct), cfg
 
 
+@pytest.mark.parametrize("m,n,k", [(1004, 1728, 6912), (1831, 1280, 5120), (307, 1792, 7168)])
+def test_fp32_products_keep_the_split_of_their_long_sums(m, n, k):
+    """A split's sums are shorter: 7.4e-7 from 64 bits in one part at K 1728, 5.3e-7 in two.  All
+    unsplit tilings add in one order (the same bits), so speed alone chooses among them."""
+    (kernel,) = _program(m, n, k, True, DType.f32).kernels
+    cands = hb._candidates(kernel)
+    first = min(cands, key=hb._rank(kernel, cands, fitted=False))
+    assert first.KSPLIT > 1 and hb.analytic_config(kernel) == first
+
+
 def test_split_launches_share_the_workspace():
     """Counters at the head of the block, as many as any launch has; partials behind them."""
     dt = DType.bf16
