@@ -664,9 +664,13 @@ class HipProgram:
 
     def __call__(self, *inputs: torch.Tensor) -> list[torch.Tensor]:
         ins = self._prepare(inputs)
-        take, dev = self.pool.take_output, self._dev
-        outs = [take(shape, dtype, dev) for shape, dtype in self._out_specs]
-        stream = _current_stream(self.device_index)
+        dev, stream = self._dev, _current_stream(self.device_index)
+        if stream and torch.cuda.is_current_stream_capturing():
+            # the captured graph's own memory, which no later call may be given
+            outs = [torch.empty(shape, dtype=dtype, device=dev) for shape, dtype in self._out_specs]
+        else:
+            take = self.pool.take_output
+            outs = [take(shape, dtype, dev, stream) for shape, dtype in self._out_specs]
         self._calls += 1
         if self.launches:
             if self.use_graph:

@@ -17,7 +17,10 @@ handle.  So a buffer is free exactly when the storage's C++ use count and the
 handle's Python reference count are back at the values measured when the pool
 created it.
 
-On the GPU the point is pointer stability: a program called in a loop whose
+On the GPU a buffer serves the stream it was first taken on: what the caller dropped there may
+still be read or written by kernels that only that stream orders.  (A program called under
+stream capture does not use the pool: its outputs belong to the captured graph's memory.)
+There the point is pointer stability: a program called in a loop whose
 results are dropped each time gets the same output addresses every call,
 so a captured hipGraph for that pointer set is replayed, not re-captured.
 """
@@ -52,7 +55,7 @@ class _Buffer:
 
 
 class BufferPool:
-    """Per (shape, dtype, device): the storages handed out so far, oldest first.
+    """Per (shape, dtype, device, stream): the storages handed out so far, oldest first.
 
     At most ``MAX_HELD`` storages are remembered per key; when a call finds all
     of them still in the caller's hands it allocates a new one and forgets the
@@ -63,10 +66,10 @@ class BufferPool:
     def __init__(self):
         self._held: dict[tuple, list[_Buffer]] = {}
 
-    def take_output(self, shape, dtype: torch.dtype, device) -> torch.Tensor:
+    def take_output(self, shape, dtype: torch.dtype, device, stream: int = 0) -> torch.Tensor:
         if type(shape) is not tuple:
             shape = tuple(int(d) for d in shape)
-        key = (shape, dtype, device)
+        key = (shape, dtype, device, stream)
         held = self._held.get(key)
         if held is None:
             held = self._held[key] = []

@@ -74,3 +74,13 @@ def test_scalar_outputs():
     p = s.data_ptr()
     del s
     assert pool.take_output((), DT, DEV).data_ptr() == p
+
+
+def test_a_dropped_buffer_stays_with_its_stream():
+    """What one stream's caller dropped may still be in use by that stream's kernels."""
+    pool = BufferPool()
+    a = pool.take_output(SHAPE, DT, DEV, 1)
+    p = a.data_ptr()
+    del a
+    b = pool.take_output(SHAPE, DT, DEV, 2)
+    assert b.data_ptr() != p and pool.take_output(SHAPE, DT, DEV, 1).data_ptr() == p

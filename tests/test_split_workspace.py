@@ -176,6 +176,29 @@ def test_replayed_program_is_recorded_in_the_callers_capture(k):
         assert all(torch.equal(o, t) and torch.equal(e, t) for o, e, t in zip(outs, eager, refs))
 
 
+def test_values_dropped_inside_a_capture_stay_the_graphs():
+    """An intermediate dropped while capturing is written again by every replay: later calls on
+    that stream, and on others, must not be given its memory."""
+    f, g = tj.jit(lambda x: x * 2.0 + 1.0, tune=False), tj.jit(lambda x: tj.sigmoid(x), tune=False)
+    x, other = torch.randn(257, 96, device=DEV), torch.randn(257, 96, device=DEV)
+    want_f, want_g = f(other).clone(), g(f(x)).clone()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        y = f(x)
+        z = g(y)
+        del y
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            kept = [f(other) for _ in range(3)]
+        kept += [f(other) for _ in range(3)]
+        torch.cuda.synchronize()
+        z.fill_(7)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(z, want_g) and all(torch.equal(k, want_f) for k in kept)
+
+
 def test_more_streams_than_blocks():
     prog, args, ref, _ = _split_program()
     outs = [torch.empty_like(ref) for _ in range(45)]
