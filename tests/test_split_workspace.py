@@ -222,8 +222,7 @@ def test_a_program_holds_one_block_until_a_second_stream_needs_one():
     """And run_static works from the static array and counters of its own, also as the program's
     first call and under capture."""
     m, n, split = 256, 4096, 4
-    torch.cuda.synchronize()
-    before = torch.cuda.mem_get_info()[0]
+    _split_program()                                     # the library's static array is in place
     args, ref = _integers(m, n, 4096, True, DT)
     out = torch.empty_like(ref)
     torch.cuda.synchronize()
